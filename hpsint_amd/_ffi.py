@@ -127,6 +127,7 @@ _SIGNATURES = {
     "hps_precond_get_blocks": [vp, vp],
     "hps_dot": [vp, i64, vp, vp, pd],
     "hps_norm2": [vp, i64, vp, pd],
+    "hps_norm2_diff": [vp, i64, vp, vp, pd],
     "hps_block_norms": [vp, vp, pd],
     "hps_axpy": [vp, i64, dbl, vp, vp],
     "hps_sadd": [vp, i64, dbl, dbl, vp, vp],
@@ -163,6 +164,9 @@ _SIGNATURES = {
     "hps_mlp_adam": [vp, cint, cint, vp, vp, vp, vp, ctypes.c_float, ctypes.c_float,
                      ctypes.c_float, ctypes.c_float, cint, vp],
     "hps_mlp_features": [vp, vp, vp, dbl, dbl, dbl, vp, vp, vp],
+    "hps_mlp_infer_workspace": [vp, ctypes.POINTER(i64)],
+    "hps_mlp_infer": [vp, vp, vp, dbl, dbl, dbl, ctypes.POINTER(vp), ctypes.POINTER(vp), vp, vp,
+                      vp, vp, vp],
     "hps_mlp_predict": [vp, vp, vp, vp, vp, vp, vp, vp],
     "hps_mlp_targets": [vp, vp, vp, vp, vp, vp, vp, vp],
 }

@@ -1075,6 +1075,15 @@ extern "C" int hps_norm2(hps_operator op, int64_t n, const double *x, double *re
   return fetch(op, 1, result);
 }
 
+extern "C" int hps_norm2_diff(hps_operator op, int64_t n, const double *x, const double *y,
+                              double *result)
+{
+  if (int r = check_op(op))
+    return r;
+  hps::blas_norm2_diff(op->stream, n, x, y, op->red_partial, op->red_out);
+  return fetch(op, 1, result);
+}
+
 extern "C" int hps_block_norms(hps_operator op, const double *x, double *result)
 {
   if (int r = check_op(op))
@@ -1372,12 +1381,9 @@ extern "C" int hps_mlp_adam(hps_operator op, int n_out, int n_in, float *W, floa
   return HPS_OK;
 }
 
-extern "C" int hps_mlp_features(hps_operator op, const double *u_prev, const double *u_cur,
-                                double dt, double dt_scale, double inc_scale, void *X, int *top2,
-                                float *lscale)
+// stencil parameters of the operator's nodes
+static hps::FeatParams feat_params(hps_operator op, double dt, double dt_scale, double inc_scale)
 {
-  if (int r = check_op(op))
-    return r;
   hps::FeatParams fp;
   fp.n_nodes = op->n_nodes;
   for (int d = 0; d < 3; ++d)
@@ -1395,7 +1401,57 @@ extern "C" int hps_mlp_features(hps_operator op, const double *u_prev, const dou
   fp.dt_scale  = dt_scale;
   fp.inc_scale = inc_scale;
   fp.inc_floor = inc_scale > 0.0 ? 1e-3 / inc_scale : 0.0;
-  hps::mlp_features(op->stream, fp, u_prev, u_cur, (uint16_t *)X, top2, lscale);
+  return fp;
+}
+
+extern "C" int hps_mlp_features(hps_operator op, const double *u_prev, const double *u_cur,
+                                double dt, double dt_scale, double inc_scale, void *X, int *top2,
+                                float *lscale)
+{
+  if (int r = check_op(op))
+    return r;
+  hps::mlp_features(op->stream, feat_params(op, dt, dt_scale, inc_scale), u_prev, u_cur,
+                    (uint16_t *)X, top2, lscale);
+  HPS_LAUNCHED();
+  return HPS_OK;
+}
+
+extern "C" int hps_mlp_infer_workspace(hps_operator op, int64_t *bytes)
+{
+  if (int r = check_op(op))
+    return r;
+  if (!bytes)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_infer_workspace: null argument");
+  *bytes = hps::mlp_infer_workspace(feat_params(op, 0.0, 0.0, 0.0));
+  return HPS_OK;
+}
+
+extern "C" int hps_mlp_infer(hps_operator op, const double *u_prev, const double *u_cur,
+                             double dt, double dt_scale, double inc_scale, const void *const *W,
+                             const float *const *b, const float *out_scale, int *top2,
+                             float *lscale, double *u_pred, void *workspace)
+{
+  if (int r = check_op(op))
+    return r;
+  if (!u_prev || !u_cur || !W || !b || !out_scale || !top2 || !lscale || !u_pred || !workspace)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_infer: null argument");
+  const uint16_t *Wl[4];
+  for (int l = 0; l < 4; ++l)
+    {
+      if (!W[l] || !b[l])
+        return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_infer: null argument");
+      Wl[l] = (const uint16_t *)W[l];
+    }
+  for (const double *u : {u_prev, u_cur})
+    if (u_pred < u + op->n_dofs && u < u_pred + op->n_dofs)
+      return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_infer: u_pred overlaps an input");
+  const hps::FeatParams fp = feat_params(op, dt, dt_scale, inc_scale);
+  if (hps::mlp_infer_workspace(fp) == 0)
+    return fail(HPS_ERR_UNSUPPORTED, "mlp_infer: mesh too large");
+  if ((uintptr_t)workspace & 15)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_infer: workspace must be 16-byte aligned");
+  hps::mlp_infer(op->stream, fp, u_prev, u_cur, Wl, b, out_scale, top2, lscale, u_pred,
+                 workspace);
   HPS_LAUNCHED();
   return HPS_OK;
 }

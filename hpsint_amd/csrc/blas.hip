@@ -49,6 +49,24 @@ namespace hps
       partial[blockIdx.x] = s;
   }
 
+  // |x - y|^2 without forming the difference in memory
+  __global__ void __launch_bounds__(RB)
+    k_diff_sq(int64_t n, const double *__restrict__ x, const double *__restrict__ y,
+              double *__restrict__ partial)
+  {
+    __shared__ double sh[RB / 64];
+    double            s = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * RB)
+      {
+        const double d = x[i] - y[i];
+        s += d * d;
+      }
+    s = block_reduce(s, sh);
+    if (threadIdx.x == 0)
+      partial[blockIdx.x] = s;
+  }
+
   // sums the RED_BLOCKS partial rows of k values each: out[j] = sum_b
   // partial[b*k + j].  Block j owns column j; thread t loads rows t, t + RB,
   // ... all at once and adds them in row order, then the wave trees and the
@@ -617,6 +635,13 @@ namespace hps
   void blas_norm2(hipStream_t s, int64_t n, const double *x, double *partial, double *out)
   {
     k_dot<<<RED_BLOCKS, RB, 0, s>>>(n, x, x, partial);
+    finish(s, 1, partial, out, 1);
+  }
+
+  void blas_norm2_diff(hipStream_t s, int64_t n, const double *x, const double *y,
+                       double *partial, double *out)
+  {
+    k_diff_sq<<<RED_BLOCKS, RB, 0, s>>>(n, x, y, partial);
     finish(s, 1, partial, out, 1);
   }
 

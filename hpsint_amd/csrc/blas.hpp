@@ -13,6 +13,8 @@ namespace hps
   void blas_dot(hipStream_t, int64_t n, const double *x, const double *y, double *partial,
                 double *out);
   void blas_norm2(hipStream_t, int64_t n, const double *x, double *partial, double *out);
+  void blas_norm2_diff(hipStream_t, int64_t n, const double *x, const double *y, double *partial,
+                       double *out);
   void blas_block_norms(hipStream_t, int64_t n_nodes, int nc, const double *x,
                         double *partial, double *out);
   void blas_multi_dot(hipStream_t, int64_t n, int k, const double *V, const double *w,

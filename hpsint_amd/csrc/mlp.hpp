@@ -37,6 +37,13 @@ namespace hps
                 uint16_t *WTb);
   void mlp_features(hipStream_t, const FeatParams &, const double *u_prev, const double *u_cur,
                     uint16_t *X, int *top2, float *lscale);
+  // features, the 272-128-128-128-4 network and u_pred (also writes top2 and
+  // lscale); out must not overlap u_prev or u_cur.  ws: mlp_infer_workspace
+  // bytes of 16-byte aligned device memory (0 bytes: mesh not covered)
+  int64_t mlp_infer_workspace(const FeatParams &);
+  void    mlp_infer(hipStream_t, const FeatParams &, const double *u_prev, const double *u_cur,
+                    const uint16_t *const *W, const float *const *b, const float *out_scale,
+                    int *top2, float *lscale, double *out, void *ws);
   void mlp_predict(hipStream_t, int64_t n_nodes, int nc, const double *u_prev,
                    const double *u_cur, const float *Y, const int *top2, const float *out_scale,
                    const float *lscale, double *u_pred);

@@ -147,20 +147,28 @@ class LearnedPredictor:
         self.out_scale = torch.tensor(list(out_scale) if out_scale is not None else [1.0] * N_OUT,
                                       dtype=torch.float32, device=dev)
         n = op.n_nodes
-        self.X = torch.empty(n, N_IN, dtype=torch.bfloat16, device=dev)
+        self._X = None
+        self._ws = None
         self.top2 = torch.empty(n, 2, dtype=torch.int32, device=dev)
         self.lscale = torch.empty(n, dtype=torch.float32, device=dev)
-        self.diff = torch.empty(op.n_dofs, dtype=torch.float64, device=dev)
         self.use_network = True
         self.inc_scale = 1.0
 
+    @property
+    def X(self):
+        """feature rows of the last features() call (allocated by the first
+        use: the fused inference keeps no rows)"""
+        if self._X is None:
+            self._X = torch.empty(self.op.n_nodes, N_IN, dtype=torch.bfloat16,
+                                  device=self.mlp.W[0].device)
+        return self._X
+
     def step_scale(self, u_prev, u_cur):
         """RMS of u_cur - u_prev, computed by the library"""
-        h = self.op.handle
         n = self.op.n_dofs
-        check(lib().hps_copy(h, n, _p(self.diff), _p(u_cur)))
-        check(lib().hps_axpy(h, n, -1.0, _p(u_prev), _p(self.diff)))
-        return max(self.op.norm(self.diff) / math.sqrt(n), 1e-300)
+        r = ctypes.c_double()
+        check(lib().hps_norm2_diff(self.op.handle, n, _p(u_cur), _p(u_prev), ctypes.byref(r)))
+        return max(r.value / math.sqrt(n), 1e-300)
 
     def features(self, u_prev, u_cur, dt):
         self.inc_scale = 1.0 / self.step_scale(u_prev, u_cur)
@@ -169,8 +177,33 @@ class LearnedPredictor:
                                      _p(self.lscale)))
         return self.X, self.top2
 
+    def _infer_workspace(self, u_prev, u_cur, out):
+        """the workspace of hps_mlp_infer, or None where that call does not
+        cover the prediction: other widths than the built network's, an
+        output that overlaps an input (its stencils read the inputs while
+        others' results are written) or a mesh beyond its 32-bit offsets"""
+        size = 8 * self.op.n_dofs
+        if (self.mlp.dims != [N_IN, 128, 128, 128, N_OUT]
+                or any(abs(out.data_ptr() - u.data_ptr()) < size for u in (u_prev, u_cur))):
+            return None
+        if self._ws is None:
+            n = ctypes.c_int64()
+            check(lib().hps_mlp_infer_workspace(self.op.handle, ctypes.byref(n)))
+            self._ws = torch.empty(n.value, dtype=torch.uint8, device=self.mlp.W[0].device)
+        return self._ws if self._ws.numel() else None
+
     def predict(self, u_prev, u_cur, dt, out):
         Y = None
+        ws = self._infer_workspace(u_prev, u_cur, out) if self.use_network else None
+        if ws is not None:
+            self.inc_scale = 1.0 / self.step_scale(u_prev, u_cur)
+            arr = ctypes.c_void_p * self.mlp.n_layers
+            check(lib().hps_mlp_infer(
+                self.op.handle, _p(u_prev), _p(u_cur), dt, self.dt_scale, self.inc_scale,
+                arr(*[w.data_ptr() for w in self.mlp.Wb]),
+                arr(*[b.data_ptr() for b in self.mlp.b]), _p(self.out_scale), _p(self.top2),
+                _p(self.lscale), _p(out), _p(ws)))
+            return out
         if self.use_network:
             X, _ = self.features(u_prev, u_cur, dt)
             Y, _ = self.mlp.forward(X, self.op.n_nodes)

@@ -186,6 +186,9 @@ int hps_precond_get_blocks(hps_operator op, double *blocks);
 int hps_dot(hps_operator op, int64_t n, const double *x, const double *y,
             double *result);
 int hps_norm2(hps_operator op, int64_t n, const double *x, double *result);
+/* ||x - y|| without forming the difference */
+int hps_norm2_diff(hps_operator op, int64_t n, const double *x, const double *y,
+                   double *result);
 /* per-component l2 norms (the block norms DynamicBlockVector::block(b).
  * l2_norm() would give): n_components results */
 int hps_block_norms(hps_operator op, const double *x, double *result);
@@ -352,6 +355,18 @@ int hps_mlp_features(hps_operator op, const double *u_prev, const double *u_cur,
 int hps_mlp_predict(hps_operator op, const double *u_prev, const double *u_cur,
                     const float *Y, const int *top2, const float *out_scale,
                     const float *lscale, double *u_pred);
+/* hps_mlp_features, the network of widths 272-128-128-128-4 (tanh hidden
+ * layers; W[l]: bf16, out x in; b[l]: FP32; W and b are host arrays of 4
+ * device pointers) and hps_mlp_predict in one call; top2 and lscale are
+ * written as by hps_mlp_features.  u_pred must not overlap u_prev or u_cur.
+ * workspace: 16-byte aligned device memory of hps_mlp_infer_workspace bytes,
+ * the call's own until its work on the stream ends (0 bytes: the mesh is too
+ * large for this call, use its parts). */
+int hps_mlp_infer_workspace(hps_operator op, int64_t *bytes);
+int hps_mlp_infer(hps_operator op, const double *u_prev, const double *u_cur, double dt,
+                  double dt_scale, double inc_scale, const void *const *W,
+                  const float *const *b, const float *out_scale, int *top2, float *lscale,
+                  double *u_pred, void *workspace);
 /* training targets: (u_next - (2 u_cur - u_prev)) / (ls * out_scale) on the
  * 4 outputs */
 int hps_mlp_targets(hps_operator op, const double *u_prev, const double *u_cur,
