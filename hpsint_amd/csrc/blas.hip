@@ -9,6 +9,7 @@
 
 #include <cstdint>
 #include <type_traits>
+#include <utility>
 
 #include "blas.hpp"
 
@@ -334,179 +335,193 @@ namespace hps
       dst[i] = inv[i] * src[i];
   }
 
-  // Inverse of every node's n_c x n_c block by Gauss-Jordan elimination with
-  // partial pivoting on [A | I], one node per thread (the result of
-  // FullMatrix::gauss_jordan in InverseComponentBlockDiagonalMatrix::
-  // do_update, I/lac/preconditioners.h:288-308)
-  template <int NC>
-  __global__ void __launch_bounds__(64)
-    k_invert_blocks(int64_t n_nodes, int64_t ist, const double *__restrict__ blocks,
-                                  double *__restrict__ inv64, float *__restrict__ inv32,
-                                  int *__restrict__ singular)
+  // f(integral_constant 0), f(1), ...: a loop whose index is a constant
+  template <typename F, int... I>
+  __device__ __forceinline__ void each_constant(std::integer_sequence<int, I...>, F &&f)
   {
-    const int64_t node = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (node >= n_nodes)
-      return;
-    // fully unrolled; the pivot row swap is done by selects, so both
-    // matrices stay in registers
-    double a[NC][NC], b[NC][NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i)
-#pragma unroll
-      for (int j = 0; j < NC; ++j)
-        {
-          a[i][j] = blocks[(node * NC + j) * NC + i]; // stored column by column
-          b[i][j] = i == j ? 1.0 : 0.0;
-        }
-#pragma unroll
-    for (int j = 0; j < NC; ++j)
-      {
-        int    r   = j;
-        double max = fabs(a[j][j]);
-#pragma unroll
-        for (int i = j + 1; i < NC; ++i)
-          if (fabs(a[i][j]) > max)
-            {
-              max = fabs(a[i][j]);
-              r   = i;
-            }
-        if (max == 0.0)
-          {
-            atomicAdd(singular, 1);
-            return;
-          }
-#pragma unroll
-        for (int i = j + 1; i < NC; ++i)
-          {
-            const bool sw = i == r;
-#pragma unroll
-            for (int k = 0; k < NC; ++k)
-              {
-                const double aj = a[j][k], ai = a[i][k], bj = b[j][k], bi = b[i][k];
-                a[j][k]         = sw ? ai : aj;
-                a[i][k]         = sw ? aj : ai;
-                b[j][k]         = sw ? bi : bj;
-                b[i][k]         = sw ? bj : bi;
-              }
-          }
-        const double hr = 1.0 / a[j][j];
-#pragma unroll
-        for (int k = 0; k < NC; ++k)
-          {
-            a[j][k] *= hr;
-            b[j][k] *= hr;
-          }
-#pragma unroll
-        for (int i = 0; i < NC; ++i)
-          {
-            if (i == j)
-              continue;
-            const double f = a[i][j];
-#pragma unroll
-            for (int k = 0; k < NC; ++k)
-              {
-                a[i][k] -= f * a[j][k];
-                b[i][k] -= f * b[j][k];
-              }
-          }
-      }
-    // inverses entry-major ([row * NC + column][node]): the apply reads
-    // each entry for consecutive nodes in one coalesced access
-    for (int i = 0; i < NC; ++i)
-      for (int j = 0; j < NC; ++j)
-        {
-          inv64[(int64_t)(i * NC + j) * ist + node] = b[i][j];
-          inv32[(int64_t)(i * NC + j) * ist + node] = (float)b[i][j];
-        }
+    (f(std::integral_constant<int, I>{}), ...);
   }
 
-  // the same inversion for larger blocks, whose two matrices do not fit in
-  // one lane's registers: a group of 16 lanes per node block, lane i holds
-  // row i of the block and of the inverse.  Partial pivoting by the largest
-  // magnitude among the rows not yet used (lowest row on ties); pivot rows
-  // are not moved, so the lane that pivots column j ends with row j of the
-  // inverse.  The normalised pivot row reaches the group through LDS.
-  // (16 groups per workgroup: the entry-major writes of the inverses cover
-  // 16 consecutive nodes)
-  template <int NC>
-  __global__ void __launch_bounds__(256)
-    k_invert_blocks_rows(int64_t n_nodes, int64_t ist, const double *__restrict__ blocks,
-                         double *__restrict__ inv64, float *__restrict__ inv32,
-                         int *__restrict__ singular)
+  // value of lane l of the lane's group of L (1, 2 or 4 adjacent lanes)
+  template <int L, int l>
+  __device__ __forceinline__ double group_bcast(double v)
   {
-    static_assert(NC <= 16, "one row per lane of a 16-lane group");
-    __shared__ double piv[16][2 * NC];
-    const int     grp  = threadIdx.x >> 4, i = threadIdx.x & 15;
-    const int64_t node = (int64_t)blockIdx.x * 16 + grp;
-    const bool    live = node < n_nodes && i < NC;
-    double        a[NC], b[NC];
-#pragma unroll
-    for (int k = 0; k < NC; ++k)
+    if constexpr (L == 1)
+      return v;
+    else
       {
-        a[k] = live ? blocks[(node * NC + k) * NC + i] : 0.0; // stored column by column
-        b[k] = k == i ? 1.0 : 0.0;
+        constexpr int ctl = L == 4 ? 0x55 * l : (l ? 0xF5 : 0xA0); // quad_perm
+        const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), ctl, 0xF, 0xF, false);
+        const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), ctl, 0xF, 0xF, false);
+        return __hiloint2double(hi, lo);
       }
-    bool used = !live; // rows of absent lanes never pivot
-    bool sing = false;
-    int  col  = 0;     // the column this lane pivoted
+  }
+
+  // Inverse of every node's n_c x n_c block by Gauss-Jordan elimination in
+  // place with partial pivoting (the result of FullMatrix::gauss_jordan in
+  // InverseComponentBlockDiagonalMatrix::do_update, I/lac/preconditioners.h:
+  // 288-308).  L lanes per node: lane l holds the columns c = L k + l in
+  // registers (one lane up to 6 components, two adjacent lanes up to 11, four
+  // above: no allocation spills at 2 waves/SIMD); the pivot column reaches the partner
+  // by DPP.  Rows are exchanged under a wave-uniform branch, which the usual
+  // diagonal pivots skip; the columns' final places are tracked as indices
+  // and applied by the store addresses.
+  // Bound: HBM (8 n_c^2 bytes read, 12 n_c^2 written per node).  Blocks come
+  // in through LDS in runs of whole columns (a lane's own columns would be
+  // read at an n_c^2 stride), and every store of a wave covers 64 / L
+  // consecutive nodes of one entry.  10 components, 1.88 M nodes: 1.94 ms
+  // with one row per lane of a 16-lane group (stores of 4 consecutive nodes,
+  // two barriers per pivot), 1.05 ms so;
+  // 12 components, 0.55 M nodes: 0.87 -> 0.56 ms.
+  template <int NC, int L>
+  __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+    k_invert_blocks(int64_t n_nodes, int64_t ist, const double *__restrict__ blocks,
+                    double *__restrict__ inv64, float *__restrict__ inv32,
+                    int *__restrict__ singular)
+  {
+    constexpr int NW = (NC + L - 1) / L; // columns per lane
+    constexpr int NN = 64 / L;           // nodes per wave
+    constexpr int KC = 2;                // columns per lane and staged run
+    constexpr int NQ = (NW + KC - 1) / KC;
+    constexpr int RP = (KC * L * NC) | 1; // staged row, odd: bank spread
+    __shared__ double sh[NN * RP];
+    const int         t = threadIdx.x, l = t % L, n = t / L;
+    const int64_t     n0 = (int64_t)blockIdx.x * NN, node = n0 + n;
+    const int         n_here = n_nodes - n0 < NN ? (int)(n_nodes - n0) : NN;
+    double            a[NC][NW];
+    // run q: the values of columns KC L q ... of one node
+    auto cols = [](int q) { return KC * L * (q + 1) <= NC ? KC * L : NC - KC * L * q; };
+    double v[NQ][KC * NC];
+    each_constant(std::make_integer_sequence<int, NQ>{}, [&](auto Q) {
+      constexpr int q = Q, run = cols(q) * NC;
 #pragma unroll
-    for (int j = 0; j < NC; ++j)
-      {
-        double v = used ? -1.0 : fabs(a[j]);
-        int    r = i;
+      for (int p = 0; p < (NN * run + 63) / 64; ++p)
+        {
+          const int i = t + 64 * p, m = i / run;
+          v[q][p]     = 0.0;
+          if (m < n_here)
+            v[q][p] = blocks[(n0 + m) * (NC * NC) + KC * L * q * NC + (i - m * run)];
+        }
+    });
+    each_constant(std::make_integer_sequence<int, NQ>{}, [&](auto Q) {
+      constexpr int q = Q, run = cols(q) * NC;
 #pragma unroll
-        for (int m = 1; m < 16; m <<= 1)
+      for (int p = 0; p < (NN * run + 63) / 64; ++p)
+        {
+          const int i = t + 64 * p, m = i / run;
+          if (m < NN)
+            sh[m * RP + (i - m * run)] = v[q][p];
+        }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < KC; ++k)
+        if (q * KC + k < NW)
+#pragma unroll
+          for (int i = 0; i < NC; ++i)
+            {
+              // (past column NC: any finite value; its results are not stored)
+              const int c          = L * k + l;
+              a[i][q * KC + k] = sh[n * RP + (c < cols(q) ? c : 0) * NC + i];
+            }
+      __syncthreads();
+    });
+    int  piv[NC];
+    bool sing = false, moved = false;
+    each_constant(std::make_integer_sequence<int, NC>{}, [&](auto J) {
+      constexpr int j   = J;
+      const bool    own = l == j % L; // holds column j
+      double        x[NC];
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+        {
+          x[i] = group_bcast<L, j % L>(a[i][j / L]);
+          // the column of the inverse grows in its place
+          a[i][j / L] = own ? (i == j ? 1.0 : 0.0) : a[i][j / L];
+        }
+      int    r   = j;
+      double max = fabs(x[j]);
+#pragma unroll
+      for (int i = j + 1; i < NC; ++i)
+        if (fabs(x[i]) > max)
           {
-            const double ov = __shfl_xor(v, m, 16);
-            const int    orr = __shfl_xor(r, m, 16);
-            if (ov > v || (ov == v && orr < r))
-              {
-                v = ov;
-                r = orr;
-              }
+            max = fabs(x[i]);
+            r   = i;
           }
-        sing         = sing || !(v > 0.0);
-        const bool me = i == r;
-        if (me)
-          {
-            const double hr = sing ? 0.0 : 1.0 / a[j];
+      sing   = sing || (NC <= 6 ? max == 0.0 : !(max > 0.0));
+      piv[j] = r;
+      if (__any(r != j))
+        {
+          moved = true;
 #pragma unroll
-            for (int k = 0; k < NC; ++k)
-              {
-                a[k] *= hr;
-                b[k] *= hr;
-                piv[grp][k]      = a[k];
-                piv[grp][NC + k] = b[k];
-              }
-            used = true;
-            col  = j;
-          }
-        __syncthreads();
-        if (!me && live)
-          {
-            const double f = a[j];
+          for (int i = j + 1; i < NC; ++i)
+            {
+              const bool sw = i == r;
+              if (!__any(sw))
+                continue;
 #pragma unroll
-            for (int k = 0; k < NC; ++k)
-              {
-                a[k] -= f * piv[grp][k];
-                b[k] -= f * piv[grp][NC + k];
-              }
-          }
-        __syncthreads();
-      }
+              for (int k = 0; k < NW; ++k)
+                {
+                  // (column j: the unit column stays, its row j is the 1)
+                  const bool   here = sw && !(own && k == j / L);
+                  const double aj = a[j][k], ai = a[i][k];
+                  a[j][k] = here ? ai : aj;
+                  a[i][k] = here ? aj : ai;
+                }
+              const double xj = x[j], xi = x[i];
+              x[j] = sw ? xi : xj;
+              x[i] = sw ? xj : xi;
+            }
+        }
+      const double p = 1.0 / x[j];
+#pragma unroll
+      for (int k = 0; k < NW; ++k)
+        a[j][k] *= p;
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+        if (i != j)
+#pragma unroll
+          for (int k = 0; k < NW; ++k)
+            a[i][k] -= x[i] * a[j][k];
+      // (keeps every pivot's updates in place: moved down to the stores,
+      // they hold all pivot columns and spill)
+#pragma unroll
+      for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int k = 0; k < NW; ++k)
+          asm volatile("" : "+v"(a[i][k]));
+    });
+    if (n >= n_here)
+      return;
     if (sing)
       {
-        if (i == 0 && node < n_nodes)
+        if (l == 0)
           atomicAdd(singular, 1);
         return;
       }
-    if (live)
+    // the inverse's columns: undo the row exchanges, last one first
+    int64_t place[NW];
 #pragma unroll
-      for (int k = 0; k < NC; ++k)
-        {
-          inv64[(int64_t)(col * NC + k) * ist + node] = b[k];
-          inv32[(int64_t)(col * NC + k) * ist + node] = (float)b[k];
-        }
+    for (int k = 0; k < NW; ++k)
+      {
+        int c = L * k + l;
+        if (moved)
+#pragma unroll
+          for (int j = NC - 1; j >= 0; --j)
+            c = c == j ? piv[j] : (c == piv[j] ? j : c);
+        place[k] = c * ist + node;
+      }
+    // entry-major ([row * NC + column][node]): the apply reads each entry
+    // for consecutive nodes in one coalesced access
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int k = 0; k < NW; ++k)
+        if (L * k + l < NC)
+          {
+            const int64_t e = (int64_t)i * NC * ist + place[k];
+            inv64[e]        = a[i][k];
+            inv32[e]        = (float)a[i][k];
+          }
   }
 
   // dst_n = B_n^-1 src_n for the nodes of a chunk of 256 NPT, thread t
@@ -840,15 +855,13 @@ namespace hps
   bool invert_blocks(hipStream_t s, int64_t n_nodes, int nc, const double *blocks,
                      double *inv64, float *inv32, int *singular)
   {
-    // up to 6 components both matrices stay in one lane's registers
-    const int g  = (int)((n_nodes + 63) / 64);
-    const int g16 = (int)((n_nodes + 15) / 16);
     const int64_t ist = inv_stride(n_nodes);
-#define HPS_CALL(N)                                                                          \
-  if constexpr (N <= 6)                                                                      \
-    k_invert_blocks<N><<<g, 64, 0, s>>>(n_nodes, ist, blocks, inv64, inv32, singular);       \
-  else                                                                                       \
-    k_invert_blocks_rows<N><<<g16, 256, 0, s>>>(n_nodes, ist, blocks, inv64, inv32, singular)
+#define HPS_CALL(N)                                                                      \
+  {                                                                                      \
+    constexpr int L = N <= 6 ? 1 : (N <= 11 ? 2 : 4);                                                    \
+    k_invert_blocks<N, L><<<(unsigned)((n_nodes * L + 63) / 64), 64, 0, s>>>(            \
+      n_nodes, ist, blocks, inv64, inv32, singular);                                     \
+  }
     HPS_NC_SWITCH(nc, HPS_CALL)
 #undef HPS_CALL
     return true;
