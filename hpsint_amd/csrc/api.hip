@@ -934,7 +934,21 @@ static int precond_update(hps_operator op, int kind, bool fp32)
                           op->stream);
           HPS_LAUNCHED();
         }
-      for (int j = 0; j < nc && !op->q2; ++j)
+      // 3D scalar mobility: every column from one pass (fe_q1_blocks.hpp);
+      // otherwise column by column
+      const bool one_pass = !op->q2 && op->dim == 3 && !op->tens && !op->cut_active &&
+                            op->ops->tx == hps::TX3 && op->ops->ty == hps::TY3;
+      if (one_pass)
+        {
+          if (!(fp32 ? hps::node_blocks_d3(op->n_grains, op->kp, op->cache32, op->blocks,
+                                           op->stream) :
+                       hps::node_blocks_d3(op->n_grains, op->kp, op->cache64, op->blocks,
+                                           op->stream)))
+            return fail(HPS_ERR_INVALID_N_COMP,
+                        "node-block Jacobi not built for this n_components");
+          HPS_LAUNCHED();
+        }
+      for (int j = 0; j < nc && !op->q2 && !one_pass; ++j)
         {
           if (fp32)
             (op->cut_active ? op->ops->probe32_cut : op->ops->probe32)(
@@ -953,7 +967,7 @@ static int precond_update(hps_operator op, int kind, bool fp32)
           else if (int r = finish_fixup<double>(op, op->blocks, nc * nc, 1, j * nc))
             return r;
         }
-      if (fp32)
+      if (fp32 && !one_pass)
         hps::blas_f32_to_f64(op->stream, nn * nc * nc, op->blocks, op->inv_blocks32);
       // cut-off: unit diagonal for the components without any entry
       if (op->cut_active && !hps::unit_empty_rows(op->stream, nn, nc, op->blocks))

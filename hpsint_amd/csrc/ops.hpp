@@ -303,6 +303,14 @@ namespace hps
                     const unsigned *masks, const float *src, const float *cache, float *dst,
                     float *part, hipStream_t s);
 
+  // node blocks (node by node, column by column) of the 3D scalar-mobility
+  // tangent without the grain cut-off, from the cache of the TX3 x TY3 tiles
+  // (fe_q1_blocks.hpp); false when n_grains is not built
+  bool node_blocks_d3(int n_grains, const KParams &kp, const double *cache, double *blocks,
+                      hipStream_t s);
+  bool node_blocks_d3(int n_grains, const KParams &kp, const float *cache, double *blocks,
+                      hipStream_t s);
+
   // the 3D scalar-mobility tangent with z-column lanes (fe_q1_zcol.hpp):
   // 8 x 8 x tz tiles, ntz1 of them along y; reads the cache of the TX3 x
   // TY3 tiles.  False when n_grains is not built for it.

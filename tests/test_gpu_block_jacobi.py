@@ -46,3 +46,36 @@ def test_inverse_of_node_blocks(G, w0):
     assert np.all(res <= bound * np.linalg.norm(y, axis=1))
     if w0 < 1.0:   # the case is what it claims: rows are exchanged
         assert np.all(np.abs(B[:, 1, 0]) > np.abs(B[:, 0, 0]))
+
+
+# windows of 7 x 7 completed nodes, marches of 4 planes or more, cache tiles
+# of 8 x 4 x 16 cells
+@pytest.mark.parametrize("cells,G", [
+    ((1, 1, 1), 1), ((6, 6, 3), 2), ((7, 13, 5), 3), ((9, 3, 17), 4), ((14, 5, 4), 5),
+    ((8, 4, 16), 6), ((5, 8, 33), 7), ((20, 15, 18), 8), ((13, 7, 2), 9), ((3, 9, 7), 10),
+    ((6, 2, 9), 11), ((8, 12, 6), 12)])
+def test_one_pass_blocks_match_column_by_column(cells, G):
+    """the cut-off operator with every order parameter active assembles the
+    same blocks by applying the tangent to one unit input per column; both
+    add the same products in other orders, at most 8 cells of 8 points"""
+    op = operator(cells, G)
+    nc = G + 2
+    blocks = torch.empty(op.n_nodes, nc, nc, dtype=torch.float64, device="cuda")
+    from hpsint_amd._ffi import check, lib
+    import ctypes
+
+    def get(fp32):
+        Preconditioner(op, "InverseComponentBlockDiagonalMatrix").do_update(fp32=fp32)
+        check(lib().hps_precond_get_blocks(op.handle, ctypes.c_void_p(blocks.data_ptr())))
+        return blocks.clone()
+
+    one64, one32 = get(False), get(True)
+    u = torch.from_numpy(np.random.default_rng(G).uniform(0, 1, op.n_dofs)).cuda()
+    op.set_grain_cut_off(1e-300)
+    op.set_component_mask(u)
+    op.fill_quadrature_point_values(u)
+    col64 = get(False)
+    scale = col64.abs().amax(dim=(1, 2), keepdim=True)
+    assert ((one64 - col64).abs() <= 64 * EPS * scale * nc).all()
+    eps32 = float(np.finfo(np.float32).eps)
+    assert ((one32 - col64).abs() <= 64 * eps32 * scale * nc).all()
