@@ -78,6 +78,11 @@ class HpsNewtonStats(ctypes.Structure):
     ]
 
 
+class HpsMlpParams(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p * 4)
+                for name in ("W", "W_bf16", "b", "mW", "vW", "mb", "vb")]
+
+
 class HpsError(RuntimeError):
     def __init__(self, code, msg):
         super().__init__("hpsint_amd error %d: %s" % (code, msg))
@@ -163,6 +168,10 @@ _SIGNATURES = {
     "hps_mlp_loss": [vp, i64, vp, vp, vp, vp, cint, ctypes.POINTER(ctypes.c_float)],
     "hps_mlp_adam": [vp, cint, cint, vp, vp, vp, vp, ctypes.c_float, ctypes.c_float,
                      ctypes.c_float, ctypes.c_float, cint, vp],
+    "hps_mlp_train_workspace": [vp, cint, ctypes.POINTER(i64)],
+    "hps_mlp_train_step": [vp, cint, vp, vp, ctypes.POINTER(HpsMlpParams), ctypes.c_float,
+                           ctypes.c_float, ctypes.c_float, ctypes.c_float, cint, vp,
+                           ctypes.POINTER(ctypes.c_float)],
     "hps_mlp_features": [vp, vp, vp, dbl, dbl, dbl, vp, vp, vp],
     "hps_mlp_infer_workspace": [vp, ctypes.POINTER(i64)],
     "hps_mlp_infer": [vp, vp, vp, dbl, dbl, dbl, ctypes.POINTER(vp), ctypes.POINTER(vp), vp, vp,

@@ -1379,6 +1379,72 @@ extern "C" int hps_mlp_loss(hps_operator op, int64_t n, const float *Y, const fl
   return HPS_OK;
 }
 
+// most rows of a training step: its loss partials fit the pinned buffer
+constexpr int TRAIN_MAX_ROWS = 64 * 2 * RED_HOST_DOUBLES;
+
+extern "C" int hps_mlp_train_workspace(hps_operator op, int M, int64_t *bytes)
+{
+  if (int r = check_op(op))
+    return r;
+  if (M < 1 || !bytes)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_train_workspace: bad arguments");
+  *bytes = M > TRAIN_MAX_ROWS ? 0 : hps::mlp_train_workspace(M, nullptr);
+  return HPS_OK;
+}
+
+extern "C" int hps_mlp_train_step(hps_operator op, int M, const void *X, const float *T,
+                                  const hps_mlp_params *prm, float lr, float beta1, float beta2,
+                                  float eps, int step, void *workspace, float *loss)
+{
+  if (int r = check_op(op))
+    return r;
+  if (M < 1 || M > TRAIN_MAX_ROWS || !X || !T || !prm || !workspace || !loss)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_train_step: bad arguments");
+  if (step < 1)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_train_step: step counts from 1");
+  hps::MlpTrain t{};
+  t.M           = M;
+  t.X           = (const uint16_t *)X;
+  t.T           = T;
+  t.ws          = workspace;
+  uintptr_t low = (uintptr_t)X | (uintptr_t)workspace;
+  for (int l = 0; l < 4; ++l)
+    {
+      if (!prm->W[l] || !prm->W_bf16[l] || !prm->b[l] || !prm->mW[l] || !prm->vW[l] ||
+          !prm->mb[l] || !prm->vb[l])
+        return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_train_step: null parameter");
+      t.W[l]  = prm->W[l];
+      t.Wb[l] = (uint16_t *)prm->W_bf16[l];
+      t.b[l]  = prm->b[l];
+      t.mW[l] = prm->mW[l];
+      t.vW[l] = prm->vW[l];
+      t.mb[l] = prm->mb[l];
+      t.vb[l] = prm->vb[l];
+      low |= (uintptr_t)t.Wb[l];
+    }
+  if (low & 15)
+    return fail(HPS_ERR_INVALID_ARGUMENT,
+                "mlp_train_step: X, W_bf16 and workspace must be 16-byte aligned");
+  t.lr  = lr;
+  t.b1  = beta1;
+  t.b2  = beta2;
+  t.eps = eps;
+  t.c1  = 1.f - std::pow(beta1, (float)step);
+  t.c2  = 1.f - std::pow(beta2, (float)step);
+  int n_loss = 0;
+  (void)hps::mlp_train_workspace(M, &n_loss);
+  const float *part = hps::mlp_train_step(op->stream, t);
+  HPS_LAUNCHED();
+  float *h = (float *)op->red_host;
+  HPS_HIP(hipMemcpyAsync(h, part, n_loss * sizeof(float), hipMemcpyDeviceToHost, op->stream));
+  HPS_HIP(hipStreamSynchronize(op->stream));
+  double s = 0.0;
+  for (int i = 0; i < n_loss; ++i)
+    s += h[i];
+  *loss = (float)s;
+  return HPS_OK;
+}
+
 extern "C" int hps_mlp_adam(hps_operator op, int n_out, int n_in, float *W, float *m1,
                             float *m2, const float *grad, float lr, float beta1, float beta2,
                             float eps, int step, void *W_bf16)

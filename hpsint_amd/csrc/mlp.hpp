@@ -44,6 +44,21 @@ namespace hps
   void    mlp_infer(hipStream_t, const FeatParams &, const double *u_prev, const double *u_cur,
                     const uint16_t *const *W, const float *const *b, const float *out_scale,
                     int *top2, float *lscale, double *out, void *ws);
+  // one Adam step of the 272-128-128-128-4 network on M rows; returns the
+  // device address of the loss' partial sums (n_loss of them).  X, Wb and ws
+  // 16-byte aligned
+  struct MlpTrain
+  {
+    int             M;
+    const uint16_t *X;
+    const float    *T;
+    float          *W[4], *b[4], *mW[4], *vW[4], *mb[4], *vb[4];
+    uint16_t       *Wb[4];
+    float           lr, b1, b2, eps, c1, c2;
+    void           *ws;
+  };
+  int64_t      mlp_train_workspace(int M, int *n_loss);
+  const float *mlp_train_step(hipStream_t, const MlpTrain &);
   void mlp_predict(hipStream_t, int64_t n_nodes, int nc, const double *u_prev,
                    const double *u_cur, const float *Y, const int *top2, const float *out_scale,
                    const float *lscale, double *u_pred);

@@ -16,7 +16,7 @@ import math
 
 import torch
 
-from ._ffi import check, lib
+from ._ffi import HpsMlpParams, check, lib
 
 N_IN = 272
 N_OUT = 4
@@ -122,7 +122,28 @@ class MLP:
                                      _p(self.vb[l]), _p(gb[l]), lr, b1, b2, eps, self.step,
                                      None))
 
+    def _train_fused(self, X, T, M, lr, b1=0.9, b2=0.999, eps=1e-8):
+        """hps_mlp_train_step, or None where it does not cover the call:
+        other widths, more rows than it takes or unaligned operands"""
+        if self.dims != [N_IN, 128, 128, 128, N_OUT]:
+            return None
+        n = ctypes.c_int64()
+        check(lib().hps_mlp_train_workspace(self.op.handle, M, ctypes.byref(n)))
+        if n.value == 0 or any(t.data_ptr() % 16 for t in [X] + self.Wb):
+            return None
+        ws = self._buf("train", (n.value,), torch.uint8)
+        p = HpsMlpParams(*[(ctypes.c_void_p * 4)(*[t.data_ptr() for t in ts])
+                           for ts in (self.W, self.Wb, self.b, self.mW, self.vW, self.mb, self.vb)])
+        loss = ctypes.c_float()
+        check(lib().hps_mlp_train_step(self.op.handle, M, _p(X), _p(T), ctypes.byref(p), lr, b1,
+                                       b2, eps, self.step + 1, _p(ws), ctypes.byref(loss)))
+        self.step += 1
+        return loss.value
+
     def train_step(self, X, T, M, lr):
+        loss = self._train_fused(X, T, M, lr)
+        if loss is not None:
+            return loss
         Y, acts = self.forward(X, M)
         loss, dY = self.loss_grad(Y, T, M)
         gW, gb = self.backward(acts, dY, M)

@@ -344,6 +344,25 @@ int hps_mlp_loss(hps_operator op, int64_t n, const float *Y, const float *T, voi
 int hps_mlp_adam(hps_operator op, int n_out, int n_in, float *W, float *m1, float *m2,
                  const float *grad, float lr, float beta1, float beta2, float eps, int step,
                  void *W_bf16);
+/* One training step of the network of widths 272-128-128-128-4 on M rows (X:
+ * M x 272 bf16, T: M x 4 FP32): forward, MSE loss, backward and Adam on all
+ * parameters, as hps_mlp_gemm, hps_mlp_loss, hps_mlp_colsum and hps_mlp_adam
+ * one after the other.  Waits for the stream and returns the loss.  X, the
+ * bf16 weights and the workspace (device memory of hps_mlp_train_workspace
+ * bytes, the call's own until it returns; 0 bytes: too many rows for this
+ * call) are 16-byte aligned. */
+typedef struct
+{
+  float *W[4];              /* out x in, FP32 master weights */
+  void  *W_bf16[4];         /* their bf16 copies (read, then refreshed) */
+  float *b[4];
+  float *mW[4], *vW[4];     /* Adam moments */
+  float *mb[4], *vb[4];
+} hps_mlp_params;
+int hps_mlp_train_workspace(hps_operator op, int M, int64_t *bytes);
+int hps_mlp_train_step(hps_operator op, int M, const void *X, const float *T,
+                       const hps_mlp_params *params, float lr, float beta1, float beta2,
+                       float eps, int step, void *workspace, float *loss);
 /* per node: 272 bf16 stencil features, the node's top-2 order parameters
  * at t_n (top2: 2 ints per node) and its local increment scale ls (lscale:
  * 1 float per node; increments are divided by it).  inc_scale = 1 / (global
