@@ -784,9 +784,24 @@ namespace hps
     for (int c = 0; c < NC; ++c)
       A[c * 64 + l] = v[c];
     __syncthreads();
-    T g[NC][DIM];
+    // value rows first (times JxW): they end the life of the history values
+    T jxw = T(kp.h_prod);
+#pragma unroll
+    for (int d = 0; d < DIM; ++d)
+      jxw *= q2_w<T>(L.t[d]);
+    T y[NC];
+    residual_values<DIM, G, TENS, OP - OP_RES0>(kp.pp, v, hist, y);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      {
+        y[c] *= jxw;
+        asm volatile("" : "+v"(y[c]));
+      }
+    // gradient rows (times JxW / h): c, mu = -kappa_c grad c,
+    // eta_i = L kappa_p grad eta_i
+    T gq[NC][DIM];
     {
-      T drow[DIM][3];
+      T drow[DIM][3], flux[DIM];
 #pragma unroll
       for (int d = 0; d < DIM; ++d)
         q2_dq_row(L.t[d], drow[d]);
@@ -794,16 +809,25 @@ namespace hps
       for (int c = 0; c < NC; ++c)
 #pragma unroll
         for (int d = 0; d < DIM; ++d)
-          g[c][d] = q2_pass(A + c * 64, L.base(d), LN::str(d), drow[d]) * inv_h[d];
-    }
-    T vr[NC], gr[NC][DIM];
-    residual_qp<DIM, G, TENS, OP - OP_RES0>(kp.pp, v, g, hist, vr, gr);
-    T jxw = T(kp.h_prod);
+          gq[c][d] = q2_pass(A + c * 64, L.base(d), LN::str(d), drow[d]) * inv_h[d];
+      if constexpr (TENS)
+        residual_grad_c_tens<DIM, G>(kp.pp, v, gq[0], gq[1], gq + 2, flux);
+      else
+        residual_grad_c_scalar<DIM, G>(kp.pp, v, gq[1], flux);
+      const T kc = -T(kp.pp.kappa_c), lkp = T(kp.pp.L) * T(kp.pp.kappa_p);
 #pragma unroll
-    for (int d = 0; d < DIM; ++d)
-      jxw *= q2_w<T>(L.t[d]);
+      for (int d = 0; d < DIM; ++d)
+        {
+          const T sd = jxw * inv_h[d];
+          gq[1][d]   = (kc * gq[0][d]) * sd;
+          gq[0][d]   = flux[d] * sd;
+#pragma unroll
+          for (int c = 2; c < NC; ++c)
+            gq[c][d] = (lkp * gq[c][d]) * sd;
+        }
+    }
     __syncthreads();
-    // integration: H takes the value rows, U and A the derivative passes
+    // integration: U and A take the derivative passes
     T scol[DIM][3], dcol[DIM][3];
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
@@ -811,13 +835,11 @@ namespace hps
         q2_s_col(L.t[d], scol[d]);
         q2_dq_col(L.t[d], dcol[d]);
       }
-    T y[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c)
       {
-        y[c]           = vr[c] * jxw;
-        U[c * 64 + l]  = gr[c][0] * (jxw * inv_h[0]);
-        A[c * 64 + l]  = gr[c][1] * (jxw * inv_h[1]);
+        U[c * 64 + l] = gq[c][0];
+        A[c * 64 + l] = gq[c][1];
       }
     __syncthreads();
 #pragma unroll
@@ -829,7 +851,7 @@ namespace hps
       {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
-          U[c * 64 + l] = gr[c][2] * (jxw * inv_h[2]);
+          U[c * 64 + l] = gq[c][2];
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -874,8 +896,10 @@ namespace hps
   }
 
   // ----------------------------------------- tangent vmult and residual
+  // (residual: at least 2 waves per SIMD, 256 registers)
   template <int DIM, int G, bool TENS, int OP, typename T>
   __global__ void __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(OP == OP_VMULT ? 1 : 2)))
     q2_apply(const Q2Params kp, const T *__restrict__ src, const double *__restrict__ old0,
              const double *__restrict__ old1, const double *__restrict__ old2,
              const T *__restrict__ cache, T *__restrict__ dst)

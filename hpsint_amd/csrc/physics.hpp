@@ -579,6 +579,67 @@ namespace hps
     residual_qp<DIM, G, false, WTD>(pp, v, g, hist, vr, gr);
   }
 
+  // gradient row of c of the residual for tensorial mobility
+  // (MobilityTensorial::apply_M, S/mobility.h:758-804) from the values at the
+  // Gauss point and the gradients gc, gmu, leg[i] of c, mu and eta_i.  One
+  // grain's pairs at a time: unrolled over all pairs at once, the divisions
+  // of 45 pairs (10 order parameters) are in flight together and the
+  // allocation needs 512 registers.
+  template <int DIM, int G, typename T>
+  __device__ __forceinline__ void residual_grad_c_tens(const PhysParams &pp, const T *v,
+                                                       const T *gc, const T *gmu,
+                                                       const T (*leg)[DIM], T *out)
+  {
+    const T  c    = v[0];
+    const T *etas = v + 2;
+    {
+      const T projector_scale = T(1.001);
+      const T phi             = phi_clamped(c);
+      const T f_vol_vap       = T(pp.Mvol) * phi + T(pp.Mvap) * (T(1.0) - phi);
+      const T fsurf = T(pp.Msurf) * T(4.0) * (c * c) * ((T(1.) - c) * (T(1.) - c));
+      T       nc[DIM];
+      unit_vector<DIM>(gc, nc);
+      const T ncmu = vdot<DIM>(nc, gmu);
+#pragma unroll
+      for (int d = 0; d < DIM; ++d)
+        out[d] = (f_vol_vap + fsurf * projector_scale) * gmu[d] - nc[d] * (fsurf * ncmu);
+    }
+    if constexpr (G > 1)
+      {
+        // S grad mu - sum eta_i eta_j f_ij e_ij (e_ij . grad mu)
+        T S = T(0.0), sum = etas[0], acc[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+          acc[d] = T(0.0);
+#pragma unroll
+        for (int i = 1; i < G; ++i)
+          {
+#pragma unroll
+            for (int j = 0; j < i; ++j)
+              {
+                T egd[DIM];
+#pragma unroll
+                for (int d = 0; d < DIM; ++d)
+                  egd[d] = leg[i][d] - leg[j][d];
+                const T k = (etas[i] * etas[j]) *
+                            (unit_vector_filter_2<DIM>(egd) * vdot<DIM>(egd, gmu));
+#pragma unroll
+                for (int d = 0; d < DIM; ++d)
+                  acc[d] += k * egd[d];
+              }
+            S += etas[i] * sum; // eta_i sum_{j < i} eta_j
+            sum += etas[i];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d)
+              asm volatile("" : "+v"(acc[d]));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
+          out[d] += (S * gmu[d] - acc[d]) * (T(2.0) * T(pp.Mgb));
+      }
+  }
+
   // gradient row of c of the residual for scalar mobility: M(c, eta) grad mu
   // (MobilityScalar::apply_M, S/mobility.h:441-472)
   template <int DIM, int G, typename T>
