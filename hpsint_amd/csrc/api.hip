@@ -80,6 +80,8 @@ struct hps_operator_s
   bool                 lin_set;
   double              *part;
   double              *red_partial, *red_out, *red_host;
+  unsigned            *red_flag; // raised by the device to red_seq (pinned)
+  unsigned             red_seq;
   double             **ptrs_dev;
   double             **ptrs_host;
   int                  precond_kind;
@@ -188,7 +190,7 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
   // the march direction; HPSINT_AMD_TILE_Y / HPSINT_AMD_TILE_M override the
   // defaults for measurements
   const int tile_y = env_int("HPSINT_AMD_TILE_Y", 4);
-  const int TZ     = env_int("HPSINT_AMD_TILE_M", 16);
+  int       TZ     = env_int("HPSINT_AMD_TILE_M", 16);
   if (TZ < 1 || TZ > 4096)
     return fail(HPS_ERR_INVALID_ARGUMENT, "HPSINT_AMD_TILE_M out of range");
   // Q1 3D z-column FP64 tangent and residual: most cache tiles per march
@@ -239,7 +241,31 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
   kp.nn[0]         = p * ncx + 1;
   kp.nn[1]         = prm->dim == 3 ? p * ncy + 1 : 1;
   kp.nn[2]         = p * ncm + 1;
-  kp.tz            = TZ;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      cus < 1)
+    {
+      (void)hipGetLastError();
+      cus = 256; // MI355X
+    }
+  // Layers per Q1 tile: 16 (fewest shared nodes) while that gives 3 tiles per
+  // CU, else the deepest of 8, 4 and (up to 4 order parameters) 2 that does,
+  // or the shallowest: small meshes are bound by the latency of a tile's
+  // march.  Tangent in us with 16 / 8 / 4 / 2 layers: 2D 160 x 80 with 2
+  // order parameters 24.8 / 16.2 / 12.8 / 10.9; 24^3 with 4 49.5 / 29.9 /
+  // 20.3 / 15.5; 40^3 with 10 80 / 50 / 40 / 44; 64^3 with 4 52.8 / 47.8 /
+  // 48.0 / 48.3, with 8 91.4 / 89.3 / 90.2 / 101; 128^3 with 4 331 / 335 /
+  // 346 / 371.
+  if (ops && !std::getenv("HPSINT_AMD_TILE_M"))
+    {
+      const int64_t cols = (int64_t)((ncx + ops->tx - 1) / ops->tx) *
+                           ((ncy + ops->ty - 1) / ops->ty);
+      const int     least = G <= 4 ? 2 : 4;
+      while (TZ > least && cols * ((ncm + TZ - 1) / TZ) < 3 * (int64_t)cus)
+        TZ /= 2;
+    }
+  kp.tz = TZ;
   if (ops)
     {
       kp.nt[0] = (ncx + ops->tx - 1) / ops->tx;
@@ -338,14 +364,6 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
       // workgroups per CU (2 run at once at 2 waves/SIMD; 128^3: two tiles,
       // 64^3: one); FP32: one (3 workgroups per CU; two tiles per march
       // left a tail)
-      int dev = 0, cus = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-          cus < 1)
-        {
-          (void)hipGetLastError();
-          cus = 256; // MI355X
-        }
       op->ntz1    = (ncy + 7) / 8;
       op->zcol_mz = TZ;
       for (int m = zm; m > 1; --m)
@@ -370,8 +388,12 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
     return cleanup_fail(e);
   if ((e = hipMalloc(&op->red_out, 64 * sizeof(double))) != hipSuccess)
     return cleanup_fail(e);
-  if ((e = hipHostMalloc(&op->red_host, RED_HOST_DOUBLES * sizeof(double))) != hipSuccess)
+  // coherent: kernels write results and the flag that the host waits for
+  if ((e = hipHostMalloc(&op->red_host, (RED_HOST_DOUBLES + 8) * sizeof(double),
+                         hipHostMallocCoherent)) != hipSuccess)
     return cleanup_fail(e);
+  op->red_flag  = reinterpret_cast<unsigned *>(op->red_host + RED_HOST_DOUBLES);
+  *op->red_flag = 0;
   if ((e = hipMalloc(&op->ptrs_dev, 32 * sizeof(double *))) != hipSuccess)
     return cleanup_fail(e);
   if ((e = hipHostMalloc(&op->ptrs_host, 32 * sizeof(double *))) != hipSuccess)
@@ -1061,15 +1083,71 @@ extern "C" int hps_precond_get_blocks(hps_operator op, double *blocks)
 }
 
 // ------------------------------------------------------------------ BLAS-1
+// waits until the device has raised the flag to red_seq.  The host polls the
+// pinned flag (a stream synchronisation takes about 10 us more); now and then
+// it asks for the stream's state, so that a failed launch ends the wait.
+static int wait_flag(hps_operator op)
+{
+  const unsigned seq = op->red_seq;
+  for (unsigned spin = 1;; ++spin)
+    {
+      if (__atomic_load_n(op->red_flag, __ATOMIC_ACQUIRE) == seq)
+        return HPS_OK;
+      if (spin % 4096 != 0)
+        continue;
+      const hipError_t e = hipStreamQuery(op->stream);
+      if (e == hipErrorNotReady)
+        {
+          (void)hipGetLastError();
+          continue;
+        }
+      if (e != hipSuccess)
+        return fail(HPS_ERR_HIP, std::string("reduction: ") + hipGetErrorString(e));
+      // all work is done: the flag is up, or the kernel did not run
+      if (__atomic_load_n(op->red_flag, __ATOMIC_ACQUIRE) == seq)
+        return HPS_OK;
+      return fail(HPS_ERR_HIP, "reduction: the result was not delivered");
+    }
+}
+
+// k <= 64 results of red_out on the host
 static int fetch(hps_operator op, int k, double *result)
 {
   HPS_LAUNCHED();
-  HPS_HIP(hipMemcpyAsync(op->red_host, op->red_out, k * sizeof(double), hipMemcpyDeviceToHost,
-                         op->stream));
-  HPS_HIP(hipStreamSynchronize(op->stream));
+  hps::publish(op->stream, k, op->red_out, op->red_host, op->red_flag, ++op->red_seq);
+  HPS_LAUNCHED();
+  if (int r = wait_flag(op))
+    return r;
   for (int i = 0; i < k; ++i)
     result[i] = op->red_host[i];
   return HPS_OK;
+}
+
+// Gram-Schmidt step of GMRES (solver.hip): h[j] = <V_j, w>, w -= sum h_j V_j,
+// *norm = |w|, w /= |w| (unless 0), with one wait
+template <typename T>
+static int gram_schmidt(hps_operator op, int64_t n, int k, const T *V, T *w, double *h,
+                        double *norm)
+{
+  hps::blas_gram_schmidt<T>(op->stream, n, k, V, w, op->red_partial, op->red_out, op->red_host,
+                            op->red_host + hps::MAXK, op->red_flag, ++op->red_seq);
+  HPS_LAUNCHED();
+  if (int r = wait_flag(op))
+    return r;
+  for (int j = 0; j < k; ++j)
+    h[j] = op->red_host[j];
+  *norm = op->red_host[hps::MAXK];
+  return HPS_OK;
+}
+int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const double *V, double *w,
+                              double *h, double *norm)
+{
+  return gram_schmidt<double>(op, n, k, V, w, h, norm);
+}
+int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const float *V, float *w,
+                              double *h, double *norm)
+{
+  return gram_schmidt<float>(op, n, k, V, w, h, norm);
 }
 
 extern "C" int hps_dot(hps_operator op, int64_t n, const double *x, const double *y,

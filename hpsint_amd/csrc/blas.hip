@@ -68,13 +68,14 @@ namespace hps
       partial[blockIdx.x] = s;
   }
 
-  // sums the RED_BLOCKS partial rows of k values each: out[j] = sum_b
-  // partial[b*k + j].  Block j owns column j; thread t loads rows t, t + RB,
-  // ... all at once and adds them in row order, then the wave trees and the
-  // waves in wave order (fixed order: deterministic).
+  // sums nb partial rows of k values each: out[j] = sum_b partial[b*k + j].
+  // Block j owns column j; thread t loads rows t, t + RB, ... all at once and
+  // adds them in row order, then the wave trees and the waves in wave order
+  // (fixed order: deterministic).
   static_assert(RED_BLOCKS % RB == 0, "finish rows per thread");
   __global__ void __launch_bounds__(RB)
-    k_finish(int k, const double *__restrict__ partial, double *__restrict__ out, int do_sqrt)
+    k_finish(int nb, int k, const double *__restrict__ partial, double *__restrict__ out,
+             int do_sqrt)
   {
     constexpr int     PER = RED_BLOCKS / RB;
     __shared__ double sh[RB / 64];
@@ -82,7 +83,10 @@ namespace hps
     double            v[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i)
-      v[i] = partial[(int64_t)(threadIdx.x + i * RB) * k + j];
+      {
+        const int r = threadIdx.x + i * RB;
+        v[i]        = r < nb ? partial[(int64_t)r * k + j] : 0.0;
+      }
     double s = 0.0;
 #pragma unroll
     for (int i = 0; i < PER; ++i)
@@ -92,9 +96,31 @@ namespace hps
       out[j] = do_sqrt ? sqrt(s) : s;
   }
 
-  static void finish(hipStream_t s, int k, const double *partial, double *out, int do_sqrt)
+  static void finish(hipStream_t s, int nb, int k, const double *partial, double *out, int do_sqrt)
   {
-    k_finish<<<k, RB, 0, s>>>(k, partial, out, do_sqrt);
+    k_finish<<<k, RB, 0, s>>>(nb, k, partial, out, do_sqrt);
+  }
+
+  // the flag after the values it announces, visible to the host
+  __device__ __forceinline__ void raise_flag(unsigned *flag, unsigned seq)
+  {
+    __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+
+  __global__ void __launch_bounds__(64)
+    k_publish(int k, const double *__restrict__ out, double *host, unsigned *flag, unsigned seq)
+  {
+    if ((int)threadIdx.x < k)
+      host[threadIdx.x] = out[threadIdx.x];
+    __syncthreads();
+    __threadfence_system();
+    if (threadIdx.x == 0)
+      raise_flag(flag, seq);
+  }
+
+  void publish(hipStream_t s, int k, const double *out, double *host, unsigned *flag, unsigned seq)
+  {
+    k_publish<<<1, 64, 0, s>>>(k, out, host, flag, seq);
   }
 
   // K values reduced over the block in one pass: per-wave shuffle trees,
@@ -176,19 +202,56 @@ namespace hps
     block_reduce_k<K>(acc, sh, partial + (int64_t)blockIdx.x * pstride + pcol);
   }
 
+  // column sums of nb <= RB partial rows of K values into out, by every block
+  // for itself: wave w takes columns w, w + 4, ... (fixed order)
+  template <int K>
+  __device__ __forceinline__ void sum_rows(const double *__restrict__ rows, int nb, double *out)
+  {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int j = wave; j < K; j += RB / 64)
+      {
+        double v[RB / 64];
+#pragma unroll
+        for (int i = 0; i < RB / 64; ++i)
+          {
+            const int r = lane + 64 * i;
+            v[i]        = r < nb ? rows[(int64_t)r * K + j] : 0.0;
+          }
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < RB / 64; ++i)
+          s += v[i];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+          s += __shfl_down(s, o, 64);
+        if (lane == 0)
+          out[j] = s;
+      }
+    __syncthreads();
+  }
+
   // w -= sum_j h[j] V_j (FP64 arithmetic, stored as T); partial sums of
-  // squares of the stored w
-  template <int K, typename T>
+  // squares of the stored w.  ROWS: h is the column sums of nb partial rows
+  // (k_mdot's), summed by every block and written to h_out by the first
+  template <int K, typename T, bool ROWS>
   __global__ void __launch_bounds__(RB)
     k_maxpy_norm(int64_t n, const T *__restrict__ V, const double *__restrict__ h,
-                 T *__restrict__ w, double *__restrict__ partial)
+                 T *__restrict__ w, double *__restrict__ partial,
+                 const double *__restrict__ rows, int nb, double *__restrict__ h_out)
   {
     constexpr int     U = unroll_for<K>();
     __shared__ double sh[RB / 64][1];
+    __shared__ double hs[ROWS ? K : 1];
     double            hk[K];
+    if constexpr (ROWS)
+      {
+        sum_rows<K>(rows, nb, hs);
+        if (blockIdx.x == 0 && threadIdx.x < K)
+          h_out[threadIdx.x] = hs[threadIdx.x];
+      }
 #pragma unroll
     for (int j = 0; j < K; ++j)
-      hk[j] = h[j];
+      hk[j] = ROWS ? hs[j] : h[j];
     double        s  = 0.0;
     const int64_t st = (int64_t)gridDim.x * RB;
     int64_t       i  = (int64_t)blockIdx.x * RB + threadIdx.x;
@@ -227,6 +290,42 @@ namespace hps
       }
     double acc[1] = {s};
     block_reduce_k<1>(acc, sh, partial + blockIdx.x);
+  }
+
+  // w /= norm (as w times 1 / norm; left alone if 0), the norm read from
+  // memory or (ROWS) from nb partial sums of squares.  The first block also
+  // sends h and the norm to the host and raises the flag.
+  template <typename T, bool ROWS>
+  __global__ void __launch_bounds__(RB)
+    k_scale_norm(int64_t n, T *__restrict__ w, const double *__restrict__ norm, int nb, int k,
+                 const double *__restrict__ h, double *host_h, double *host_norm, unsigned *flag,
+                 unsigned seq)
+  {
+    __shared__ double sh[1];
+    double            v;
+    if constexpr (ROWS)
+      {
+        sum_rows<1>(norm, nb, sh);
+        v = sqrt(sh[0]);
+      }
+    else
+      v = norm[0];
+    if (blockIdx.x == 0)
+      {
+        if ((int)threadIdx.x < k)
+          host_h[threadIdx.x] = h[threadIdx.x];
+        if (threadIdx.x == 0)
+          *host_norm = v;
+        __syncthreads();
+        __threadfence_system();
+        if (threadIdx.x == 0)
+          raise_flag(flag, seq);
+      }
+    if (v == 0.0)
+      return;
+    const double a = 1.0 / v;
+    for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
+      w[i] = (T)(a * (double)w[i]);
   }
 
   // y (FP64) += sum_j a_j X_j (storage T), j < K
@@ -643,28 +742,32 @@ namespace hps
   void blas_dot(hipStream_t s, int64_t n, const double *x, const double *y,
                 double *partial, double *out)
   {
-    k_dot<<<RED_BLOCKS, RB, 0, s>>>(n, x, y, partial);
-    finish(s, 1, partial, out, 0);
+    const int nb = red_blocks(n);
+    k_dot<<<nb, RB, 0, s>>>(n, x, y, partial);
+    finish(s, nb, 1, partial, out, 0);
   }
 
   void blas_norm2(hipStream_t s, int64_t n, const double *x, double *partial, double *out)
   {
-    k_dot<<<RED_BLOCKS, RB, 0, s>>>(n, x, x, partial);
-    finish(s, 1, partial, out, 1);
+    const int nb = red_blocks(n);
+    k_dot<<<nb, RB, 0, s>>>(n, x, x, partial);
+    finish(s, nb, 1, partial, out, 1);
   }
 
   void blas_norm2_diff(hipStream_t s, int64_t n, const double *x, const double *y,
                        double *partial, double *out)
   {
-    k_diff_sq<<<RED_BLOCKS, RB, 0, s>>>(n, x, y, partial);
-    finish(s, 1, partial, out, 1);
+    const int nb = red_blocks(n);
+    k_diff_sq<<<nb, RB, 0, s>>>(n, x, y, partial);
+    finish(s, nb, 1, partial, out, 1);
   }
 
   void blas_block_norms(hipStream_t s, int64_t n_nodes, int nc, const double *x,
                         double *partial, double *out)
   {
-    k_block_sq<<<RED_BLOCKS, RB, 0, s>>>(n_nodes, nc, x, partial);
-    finish(s, nc, partial, out, 1);
+    const int nb = red_blocks(n_nodes);
+    k_block_sq<<<nb, RB, 0, s>>>(n_nodes, nc, x, partial);
+    finish(s, nb, nc, partial, out, 1);
   }
 
 #define HPS_K_SWITCH(k, CALL)                                                  \
@@ -687,29 +790,86 @@ namespace hps
   // rows in passes of at most 16 (beyond that the compiler serialises the
   // row loads of one step and the kernel drops to half bandwidth)
   template <typename T>
-  static void multi_dot_any(hipStream_t s, int64_t n, int k, const T *V, const T *w,
-                            double *partial, double *out)
+  static void multi_dot_partials(hipStream_t s, int nb, int64_t n, int k, const T *V, const T *w,
+                                 double *partial)
   {
     for (int j0 = 0; j0 < k; j0 += 16)
       {
         const int kk = k - j0 < 16 ? k - j0 : 16;
         const T  *Vj = V + (int64_t)j0 * n;
-#define HPS_CALL(K) k_mdot<K, T><<<RED_BLOCKS, RB, 0, s>>>(n, Vj, w, partial, k, j0)
+#define HPS_CALL(K) k_mdot<K, T><<<nb, RB, 0, s>>>(n, Vj, w, partial, k, j0)
         HPS_K_SWITCH(kk, HPS_CALL)
 #undef HPS_CALL
       }
-    finish(s, k, partial, out, 0);
+  }
+
+  template <typename T>
+  static void multi_dot_any(hipStream_t s, int64_t n, int k, const T *V, const T *w,
+                            double *partial, double *out)
+  {
+    const int nb = red_blocks(n);
+    multi_dot_partials<T>(s, nb, n, k, V, w, partial);
+    finish(s, nb, k, partial, out, 0);
   }
 
   template <typename T>
   static void multi_axpy_norm_any(hipStream_t s, int64_t n, int k, const T *V,
                                   const double *h, T *w, double *partial, double *out)
   {
-#define HPS_CALL(K) k_maxpy_norm<K, T><<<RED_BLOCKS, RB, 0, s>>>(n, V, h, w, partial)
+    const int nb = red_blocks(n);
+#define HPS_CALL(K)                                                                 \
+  k_maxpy_norm<K, T, false><<<nb, RB, 0, s>>>(n, V, h, w, partial, nullptr, 0, nullptr)
     HPS_K_SWITCH(k, HPS_CALL)
 #undef HPS_CALL
-    finish(s, 1, partial, out, 1);
+    finish(s, nb, 1, partial, out, 1);
   }
+
+  // Blocks up to which a Gram-Schmidt step sums the partial rows in the
+  // consuming kernels (every block again) instead of in finish kernels: three
+  // launches instead of five.  256 blocks (131 k entries): each block then
+  // reads at most 64 KB of partial sums.
+  constexpr int GS_INLINE_BLOCKS = 256;
+
+  template <typename T>
+  void blas_gram_schmidt(hipStream_t s, int64_t n, int k, const T *V, T *w, double *partial,
+                         double *out, double *host_h, double *host_norm, unsigned *flag,
+                         unsigned seq)
+  {
+    const int  nb  = red_blocks(n);
+    const bool inl = nb <= GS_INLINE_BLOCKS;
+    multi_dot_partials<T>(s, nb, n, k, V, w, partial);
+    // the norm's partial sums follow the dots'
+    double *pn = partial + (int64_t)nb * k;
+    if (inl)
+      {
+#define HPS_CALL(K) \
+  k_maxpy_norm<K, T, true><<<nb, RB, 0, s>>>(n, V, nullptr, w, pn, partial, nb, out)
+        HPS_K_SWITCH(k, HPS_CALL)
+#undef HPS_CALL
+      }
+    else
+      {
+        finish(s, nb, k, partial, out, 0);
+        pn = partial;
+#define HPS_CALL(K) \
+  k_maxpy_norm<K, T, false><<<nb, RB, 0, s>>>(n, V, out, w, pn, nullptr, 0, nullptr)
+        HPS_K_SWITCH(k, HPS_CALL)
+#undef HPS_CALL
+        finish(s, nb, 1, pn, out + MAXK, 1);
+      }
+    const int g = inl ? nb : grid_for(n, 256 * 4);
+    if (inl)
+      k_scale_norm<T, true><<<g, RB, 0, s>>>(n, w, pn, nb, k, out, host_h, host_norm, flag, seq);
+    else
+      k_scale_norm<T, false>
+        <<<g, RB, 0, s>>>(n, w, out + MAXK, nb, k, out, host_h, host_norm, flag, seq);
+  }
+  template void blas_gram_schmidt<double>(hipStream_t, int64_t, int, const double *, double *,
+                                          double *, double *, double *, double *, unsigned *,
+                                          unsigned);
+  template void blas_gram_schmidt<float>(hipStream_t, int64_t, int, const float *, float *,
+                                         double *, double *, double *, double *, unsigned *,
+                                         unsigned);
 
   void blas_multi_dot(hipStream_t s, int64_t n, int k, const double *V, const double *w,
                       double *partial, double *out)
@@ -945,8 +1105,9 @@ namespace hps
 
   void blas_norm2_f32(hipStream_t s, int64_t n, const float *x, double *partial, double *out)
   {
-    k_norm_f32<<<RED_BLOCKS, RB, 0, s>>>(n, x, partial);
-    finish(s, 1, partial, out, 1);
+    const int nb = red_blocks(n);
+    k_norm_f32<<<nb, RB, 0, s>>>(n, x, partial);
+    finish(s, nb, 1, partial, out, 1);
   }
 
   void blas_scale_f32(hipStream_t s, int64_t n, double a, float *x)

@@ -7,8 +7,18 @@
 
 namespace hps
 {
-  constexpr int RED_BLOCKS = 2048; // fixed reduction grid (deterministic sums)
+  constexpr int RED_BLOCKS = 2048; // most blocks of a reduction
   constexpr int MAXK       = 32;   // max vectors of one multi-dot
+
+  // blocks of a reduction over n entries: a function of n alone (sums are
+  // deterministic); two entries per thread of 256 until the grid is full
+  // (52 k entries, 16 vectors: 20.6 us with 2048 blocks, most of it the block
+  // trees of empty blocks)
+  inline int red_blocks(int64_t n)
+  {
+    const int64_t b = (n + 511) / 512;
+    return b < 1 ? 1 : (b > RED_BLOCKS ? RED_BLOCKS : (int)b);
+  }
 
   void blas_dot(hipStream_t, int64_t n, const double *x, const double *y, double *partial,
                 double *out);
@@ -21,6 +31,16 @@ namespace hps
                       double *partial, double *out);
   void blas_multi_axpy_norm(hipStream_t, int64_t n, int k, const double *V, const double *h,
                             double *w, double *partial, double *out);
+  // One classical Gram-Schmidt step: h[j] = <V_j, w>, w -= sum h_j V_j,
+  // norm = |w|, w /= norm (left alone if 0).  h (k values), norm and then
+  // *flag = seq are written to pinned host memory; scratch: partial (RED_BLOCKS x
+  // k values) and out (MAXK + 8)
+  template <typename T>
+  void blas_gram_schmidt(hipStream_t, int64_t n, int k, const T *V, T *w, double *partial,
+                         double *out, double *host_h, double *host_norm, unsigned *flag,
+                         unsigned seq);
+  // k <= 64 results from device memory to pinned host memory, then *flag = seq
+  void publish(hipStream_t, int k, const double *out, double *host, unsigned *flag, unsigned seq);
   void blas_axpy(hipStream_t, int64_t n, double a, const double *x, double *y);
   void blas_sadd(hipStream_t, int64_t n, double s, double a, const double *x, double *y);
   void blas_scale(hipStream_t, int64_t n, double a, double *x);

@@ -36,6 +36,12 @@ struct hps_newton_s
 
 // error reporting shared with the operator entry points (api.hip)
 int hps_internal_fail(int code, const char *msg);
+// one Gram-Schmidt step with one wait (api.hip): h[j] = <V_j, w>, w -= sum h_j
+// V_j, *norm = |w|, w /= |w| (unless 0)
+int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const double *V, double *w,
+                              double *h, double *norm);
+int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const float *V, float *w,
+                              double *h, double *norm);
 
 namespace
 {
@@ -126,6 +132,31 @@ namespace
     }
   };
 
+  // Classical Gram-Schmidt against k vectors with one re-orthogonalisation
+  // pass when the new vector loses more than half of its norm: h, the norm,
+  // and w normalised (unless its norm is 0).  The second pass starts from the
+  // normalised vector, so its coefficients and norm scale by the first norm.
+  template <typename T>
+  int orthogonalise(hps_operator op, int64_t n, int k, const T *V, T *w, double *h,
+                    double *norm)
+  {
+    HPS_TRY(hps_internal_gram_schmidt(op, n, k, V, w, h, norm));
+    // norm before the projection, sqrt(|w'|^2 + |h|^2) (V orthonormal)
+    double hh = 0.0;
+    for (int i = 0; i < k; ++i)
+      hh += h[i] * h[i];
+    if (*norm > 0.0 && *norm < 0.5 * std::sqrt(*norm * *norm + hh))
+      {
+        std::vector<double> h2(k);
+        double              n2 = 0.0;
+        HPS_TRY(hps_internal_gram_schmidt(op, n, k, V, w, h2.data(), &n2));
+        for (int i = 0; i < k; ++i)
+          h[i] += *norm * h2[i];
+        *norm *= n2;
+      }
+    return HPS_OK;
+  }
+
   // Restarted GMRES(m) with left preconditioning and classical Gram-Schmidt
   // (one re-orthogonalisation pass when the new vector loses more than
   // half of its norm); convergence as deal.II's ReductionControl on the
@@ -173,21 +204,8 @@ namespace
           {
             double *vj1 = V + (int64_t)(j + 1) * n;
             HPS_TRY(apply_prec_op(nt, V + (int64_t)j * n, vj1));
-            HPS_TRY(hps_multi_dot(op, n, j + 1, V, vj1, a.h.data()));
             double wnorm = 0.0;
-            HPS_TRY(hps_multi_axpy_norm(op, n, j + 1, V, a.h.data(), vj1, &wnorm));
-            // norm before the projection, sqrt(|w'|^2 + |h|^2) (V orthonormal)
-            double hh = 0.0;
-            for (int i = 0; i <= j; ++i)
-              hh += a.h[i] * a.h[i];
-            if (wnorm < 0.5 * std::sqrt(wnorm * wnorm + hh))
-              {
-                std::vector<double> h2(j + 1);
-                HPS_TRY(hps_multi_dot(op, n, j + 1, V, vj1, h2.data()));
-                HPS_TRY(hps_multi_axpy_norm(op, n, j + 1, V, h2.data(), vj1, &wnorm));
-                for (int i = 0; i <= j; ++i)
-                  a.h[i] += h2[i];
-              }
+            HPS_TRY(orthogonalise(op, n, j + 1, V, vj1, a.h.data(), &wnorm));
             a.h[j + 1]       = wnorm;
             const double res = a.add_column(j);
             ++it;
@@ -202,7 +220,6 @@ namespace
                 ++j;
                 break;
               }
-            HPS_TRY(hps_scale(op, n, 1.0 / wnorm, vj1));
           }
         // back substitution H y = g, x += V y
         a.solve(j);
@@ -268,20 +285,8 @@ namespace
             float *vj1 = V + (int64_t)(j + 1) * n;
             HPS_TRY(hps_vmult_f32(op, nt->y32, V + (int64_t)j * n));
             HPS_TRY(hps_precond_apply_f32(op, vj1, nt->y32));
-            HPS_TRY(hps_multi_dot_f32(op, n, j + 1, V, vj1, a.h.data()));
             double wnorm = 0.0;
-            HPS_TRY(hps_multi_axpy_norm_f32(op, n, j + 1, V, a.h.data(), vj1, &wnorm));
-            double hh = 0.0;
-            for (int i = 0; i <= j; ++i)
-              hh += a.h[i] * a.h[i];
-            if (wnorm < 0.5 * std::sqrt(wnorm * wnorm + hh))
-              {
-                std::vector<double> h2(j + 1);
-                HPS_TRY(hps_multi_dot_f32(op, n, j + 1, V, vj1, h2.data()));
-                HPS_TRY(hps_multi_axpy_norm_f32(op, n, j + 1, V, h2.data(), vj1, &wnorm));
-                for (int i = 0; i <= j; ++i)
-                  a.h[i] += h2[i];
-              }
+            HPS_TRY(orthogonalise(op, n, j + 1, V, vj1, a.h.data(), &wnorm));
             a.h[j + 1]       = wnorm;
             const double res = a.add_column(j);
             ++it;
@@ -296,7 +301,6 @@ namespace
                 ++j;
                 break;
               }
-            HPS_TRY(hps_scale_f32(op, n, 1.0 / wnorm, vj1));
           }
         a.solve(j);
         HPS_TRY(hps_axpy_multi_f32(op, n, j, a.y.data(), V, x));
