@@ -289,6 +289,7 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
   kp.pp.L       = prm->L;
   kp.pp.w0      = 0.0;
   kp.pp.w_alg   = 1.0;
+  hps::phys_derive(kp.pp);
   kp.order      = 0;
   hps::set_fold_scales(kp, prm->dim);
 

@@ -52,7 +52,7 @@ namespace hps
     double inv_h[3];  // 1/h along the physical directions x, y, z
     double jxw;       // prod(h) * (1/2)^DIM
     double w_hist[3]; // BDF weights[1..order]
-    PhysParams pp;
+    PhysProducts pp;
     // uniform scales of the folded scalar tangent for the rescaled
     // butterflies (FoldScales, set by set_fold_scales; sa = (1+1/sqrt3)/2):
     // JxW/h^2 sa^(2 DIM - 2), times -kappa_c, times L kappa_p;

@@ -597,7 +597,7 @@ namespace hps
               lin[f] = lin_e[f];
             else
               lin[f] = L.valid ? cl[f * LP] : T(0);
-          tangent_values<DIM, G, TENS>(kp.pp, lin, v, vr);
+          tangent_values<DIM, G, TENS, EL>(kp.pp, lin, v, vr);
           tangent_grad_c<DIM, G, TENS>(kp.pp, lin, v, g0, g1, gc0, qsum);
         }
       else
@@ -609,7 +609,7 @@ namespace hps
               lin[f] = lin_e[f];
             else
               lin[f] = L.valid ? cl[f * LP] : T(0);
-          tangent_values<DIM, G, TENS>(kp.pp, lin, v, vr);
+          tangent_values<DIM, G, TENS, EL>(kp.pp, lin, v, vr);
           tangent_grad_c<DIM, G, TENS>(kp.pp, lin, v, g0, g1, gc0);
         }
 #pragma unroll

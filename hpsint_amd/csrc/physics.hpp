@@ -8,9 +8,10 @@
 //   S/operator_sintering_generic.h:104-190 (tangent QP operator)
 //   S/operator_sintering_generic.h:254-308 (residual QP operator)
 // with S/ = applications/sintering/include/pf-applications/sintering/ and
-// I/ = include/pf-applications/.  Operation order follows the reference
-// expressions so that the thresholds (phi clamp, unit_vector tolerances,
-// fsurf mask) see the same values.
+// I/ = include/pf-applications/.  Where a threshold decides (phi clamp,
+// unit_vector tolerances, fsurf mask) the operation order follows the
+// reference's expressions, so that it sees the same values; polynomials
+// without one are collected to need fewer operations.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -23,6 +24,54 @@ namespace hps
     double Mvol, Mvap, Msurf, Mgb, L;
     double w0, w_alg;
   };
+
+  // PhysParams with the products that the pointwise operators use (the Q1
+  // kernels' parameters; the Q2 tile march, at its register limits, is slower
+  // with the longer argument block and forms them itself)
+  struct PhysProducts : PhysParams
+  {
+    double A2, A12, A2B2, B12, BL12, BL24; // 2 A, 12 A, 2 A + 2 B, 12 B, 12 B L, 24 B L
+    double dM, dM30, Ms4, Ms8, Mgb2;       // Mvol - Mvap, 30 times it, 4 Msurf, 8 Msurf, 2 Mgb
+  };
+#define HPS_PRODUCT(NAME, EXPR)                                            \
+  template <typename T>                                                    \
+  __host__ __device__ __forceinline__ T pp_##NAME(const PhysParams &p)     \
+  {                                                                        \
+    return T(EXPR);                                                        \
+  }                                                                        \
+  template <typename T>                                                    \
+  __host__ __device__ __forceinline__ T pp_##NAME(const PhysProducts &p)   \
+  {                                                                        \
+    return T(p.NAME);                                                      \
+  }
+  HPS_PRODUCT(A2, 2.0 * p.A)
+  HPS_PRODUCT(A12, 12.0 * p.A)
+  HPS_PRODUCT(A2B2, 2.0 * p.A + 2.0 * p.B)
+  HPS_PRODUCT(B12, 12.0 * p.B)
+  HPS_PRODUCT(BL12, 12.0 * p.B * p.L)
+  HPS_PRODUCT(BL24, 24.0 * p.B * p.L)
+  HPS_PRODUCT(dM, p.Mvol - p.Mvap)
+  HPS_PRODUCT(dM30, 30.0 * (p.Mvol - p.Mvap))
+  HPS_PRODUCT(Ms4, 4.0 * p.Msurf)
+  HPS_PRODUCT(Ms8, 8.0 * p.Msurf)
+  HPS_PRODUCT(Mgb2, 2.0 * p.Mgb)
+#undef HPS_PRODUCT
+
+  inline void phys_derive(PhysProducts &p)
+  {
+    const PhysParams &b = p;
+    p.A2                = pp_A2<double>(b);
+    p.A12               = pp_A12<double>(b);
+    p.A2B2              = pp_A2B2<double>(b);
+    p.B12               = pp_B12<double>(b);
+    p.BL12              = pp_BL12<double>(b);
+    p.BL24              = pp_BL24<double>(b);
+    p.dM                = pp_dM<double>(b);
+    p.dM30              = pp_dM30<double>(b);
+    p.Ms4               = pp_Ms4<double>(b);
+    p.Ms8               = pp_Ms8<double>(b);
+    p.Mgb2              = pp_Mgb2<double>(b);
+  }
 
   template <typename T>
   __device__ __forceinline__ T dmax(T a, T b)
@@ -177,45 +226,46 @@ namespace hps
     T kj[3], kmu[3], keta[3], gsj[3];
   };
 
+  // scalar mobility (MobilityScalar::apply_M, S/mobility.h:441-472) from p = c
+  // (1 - c) and sum_{j < i} eta_i eta_j
+  template <typename T, typename PP>
+  __device__ __forceinline__ T scalar_mobility(const PP &pp, T c, T p, T pairs)
+  {
+    return T(pp.Mvap) + pp_dM<T>(pp) * phi_clamped(c) + pp_Ms4<T>(pp) * (p * p) + pp_Mgb2<T>(pp) * pairs;
+  }
+
   // c-row coefficients of the scalar-mobility tangent
   // (MobilityScalar::apply_M_derivative, S/mobility.h:477-534):
   //   grad row of c = M grad(dmu) + s grad(mu_lin),
-  //   s = dM/dc dc + 2 Mgb sum_i (sum_j eta_j - eta_i) deta_i
-  template <int G, typename T>
-  __device__ __forceinline__ void scalar_mobility_terms(const PhysParams &pp, T c,
+  //   s = dM/dc dc + 2 Mgb sum_i (sum_j eta_j - eta_i) deta_i,
+  //   dM/dc = 30 (Mvol - Mvap) p^2 + 8 Msurf p (1 - 2 c), p = c (1 - c).
+  // The sums over pairs and over j != i are formed from running sums, O(G).
+  template <int G, typename T, typename PP>
+  __device__ __forceinline__ void scalar_mobility_terms(const PP &pp, T c,
                                                         const T *etas, const T *v, T &M,
                                                         T &s)
   {
-    const T Mvol  = T(pp.Mvol);
-    const T Mvap  = T(pp.Mvap);
-    const T Msurf = T(pp.Msurf);
-    const T Mgb   = T(pp.Mgb);
-    T       eta_sum = T(0.0), eta_ij_sum = T(0.0);
+    // (no order parameter is active in some tiles of the cut-off: G = 0)
+    T sum = G > 0 ? etas[0] : T(0.0), sv = G > 0 ? v[2] : T(0.0);
+    T ev = sum * sv, pairs = T(0.0);
 #pragma unroll
-    for (int i = 0; i < G; ++i)
+    for (int i = 1; i < G; ++i)
       {
-        eta_sum += etas[i];
-#pragma unroll
-        for (int j = 0; j < i; ++j)
-          eta_ij_sum += etas[i] * etas[j];
+        pairs += etas[i] * sum;
+        sum += etas[i];
+        ev += etas[i] * v[2 + i];
+        sv += v[2 + i];
       }
-    const T phi = phi_clamped(c);
-    M           = Mvol * phi + Mvap * (T(1.0) - phi) +
-        Msurf * T(4.0) * c * c * (T(1.0) - c) * (T(1.0) - c) + (T(2.0) * Mgb) * eta_ij_sum;
-    const T dphidc = T(30.0) * c * c * (T(1.0) - c) * (T(1.0) - c);
-    const T dMdc   = Mvol * dphidc - Mvap * dphidc +
-                   Msurf * T(8.0) * c * (T(1.0) - T(3.0) * c + T(2.0) * c * c);
-    T factor = T(0.0);
-#pragma unroll
-    for (int i = 0; i < G; ++i)
-      factor += (eta_sum - etas[i]) * v[2 + i];
-    s = dMdc * v[0] + (T(2.0) * Mgb) * factor;
+    const T p    = c * (T(1.0) - c);
+    M            = scalar_mobility(pp, c, p, pairs);
+    const T dMdc = p * (pp_dM30<T>(pp) * p + pp_Ms8<T>(pp) * (T(1.0) - T(2.0) * c));
+    s            = dMdc * v[0] + pp_Mgb2<T>(pp) * (sum * sv - ev);
   }
 
   // qsum (optional, tensorial only): sum_i deta_i Q_i formed by the caller,
   // which then need not hold the Q_i fields of lin
-  template <int DIM, int G, bool TENS, bool VALS, bool GRADC, typename T>
-  __device__ __forceinline__ void tangent_qp_rows(const PhysParams &pp,
+  template <int DIM, int G, bool TENS, bool VALS, bool GRADC, typename T, typename PP>
+  __device__ __forceinline__ void tangent_qp_rows(const PP &pp,
                                                   const T          *lin,
                                                   const T          *v,
                                                   const T (*g)[DIM],
@@ -227,20 +277,12 @@ namespace hps
     const T  c      = lin[CL::c];
     const T *etas   = lin + CL::eta;
     const T *lmu    = lin + CL::grad_mu;
-    const T  A      = T(pp.A);
-    const T  B      = T(pp.B);
     const T  L      = T(pp.L);
     const T  w0     = T(pp.w0);
     const T  Mvol   = T(pp.Mvol);
     const T  Mvap   = T(pp.Mvap);
     const T  Msurf  = T(pp.Msurf);
     const T  Mgb    = T(pp.Mgb);
-
-    // FreeEnergy EnergySecond evaluation: only the power-2 sum
-    T S2 = T(0.0);
-#pragma unroll
-    for (int i = 0; i < G; ++i)
-      S2 += etas[i] * etas[i];
 
     // 1) c row
     vr[0] = v[0] * w0;
@@ -354,6 +396,62 @@ namespace hps
         gr[i + 2][d] = Lkp * g[i + 2][d];
     if constexpr (!VALS)
       return;
+    // Value rows with the derivatives of the free energy
+    // (S/free_energy.h:37-176, 234-252) collected by powers of eta_i:
+    //   f_cc = 12 A c (c - 1) + 2 A + 2 B,  f_c,eta_i = 12 B eta_i (eta_i - 1),
+    //   f_eta_i,eta_i = 12 B (1 - c + S2) + 24 B (c - 2) eta_i + 24 B eta_i^2,
+    //   f_eta_i,eta_j = 24 B eta_i eta_j;
+    // the eta_i^2 part of the diagonal is the j = i term of
+    // 24 B eta_i sum_j eta_j deta_j, so a row costs four operations:
+    //   (b eta_i + a) deta_i + eta_i (c0 eta_i + 24 B L sum_j eta_j deta_j - c0),
+    //   a = w0 + 12 B L (1 - c + S2), b = 24 B L (c - 2), c0 = 12 B L dc
+    const T e0 = G > 0 ? etas[0] : T(0.0);
+    T       w = G > 0 ? e0 * v[2] : T(0.0), S2 = e0 * e0, ev = w, e2v = e0 * w;
+#pragma unroll
+    for (int i = 1; i < G; ++i)
+      {
+        S2 += etas[i] * etas[i];
+        w = etas[i] * v[2 + i];
+        ev += w;
+        e2v += etas[i] * w;
+      }
+    const T fcc = pp_A12<T>(pp) * (c * (c - T(1.0))) + pp_A2B2<T>(pp);
+    vr[1]       = T(pp.w_alg) * v[1] - fcc * v[0] - pp_B12<T>(pp) * (e2v - ev);
+    const T a = w0 + pp_BL12<T>(pp) * ((T(1.0) - c) + S2), b = pp_BL24<T>(pp) * (c - T(2.0));
+    const T c0 = pp_BL12<T>(pp) * v[0], f0 = pp_BL24<T>(pp) * ev - c0;
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      vr[i + 2] = (b * etas[i] + a) * v[i + 2] + etas[i] * (c0 * etas[i] + f0);
+  }
+
+  template <int DIM, int G, bool TENS, typename T, typename PP>
+  __device__ __forceinline__ void tangent_qp(const PP &pp, const T *lin, const T *v,
+                                             const T (*g)[DIM], T *vr, T (*gr)[DIM])
+  {
+    tangent_qp_rows<DIM, G, TENS, true, true>(pp, lin, v, g, vr, gr);
+  }
+
+  // ------------------------------------------------------------------
+  // The tangent split by output: the value rows need the increment's values
+  // only; the gradient row of c needs the gradients of c and mu; the other
+  // gradient rows are multiples of one input gradient each.  Kernels that
+  // stream one component at a time use these pieces; tangent_qp above is
+  // their composition.
+  // ------------------------------------------------------------------
+  // The value rows term by term (S/operator_sintering_generic.h:104-190),
+  // with more operations than the collected form of tangent_qp_rows: the FP64
+  // Q2 tile march waits for memory, not for the VALU, and is scheduled better
+  // with them (96^3, 10 order parameters, tensorial: 3.42 against 3.58 ms).
+  template <int G, typename T, typename PP>
+  __device__ __forceinline__ void tangent_values_by_term(const PP &pp, T c, const T *etas,
+                                                         const T *v, T *vr)
+  {
+    const T A = T(pp.A), B = T(pp.B), L = T(pp.L), w0 = T(pp.w0);
+    T       S2 = T(0.0);
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      S2 += etas[i] * etas[i];
+    vr[0] = v[0] * w0;
     const T d2f_dc2 = T(2.0) * A * (c * c) + T(4.0) * A * c * (T(2.0) * c - T(2.0)) +
                       T(2.0) * A * ((-c + T(1.0)) * (-c + T(1.0))) + T(2.0) * B;
     T vmu = T(pp.w_alg) * v[1] - d2f_dc2 * v[0];
@@ -389,24 +487,16 @@ namespace hps
       }
   }
 
-  template <int DIM, int G, bool TENS, typename T>
-  __device__ __forceinline__ void tangent_qp(const PhysParams &pp, const T *lin, const T *v,
-                                             const T (*g)[DIM], T *vr, T (*gr)[DIM])
-  {
-    tangent_qp_rows<DIM, G, TENS, true, true>(pp, lin, v, g, vr, gr);
-  }
-
-  // ------------------------------------------------------------------
-  // The tangent split by output: the value rows need the increment's values
-  // only; the gradient row of c needs the gradients of c and mu; the other
-  // gradient rows are multiples of one input gradient each.  Kernels that
-  // stream one component at a time use these pieces; tangent_qp above is
-  // their composition.
-  // ------------------------------------------------------------------
-  template <int DIM, int G, bool TENS, typename T>
-  __device__ __forceinline__ void tangent_values(const PhysParams &pp, const T *lin,
+  // BY_TERM: tangent_values_by_term
+  template <int DIM, int G, bool TENS, bool BY_TERM = false, typename T, typename PP>
+  __device__ __forceinline__ void tangent_values(const PP &pp, const T *lin,
                                                  const T *v, T *vr)
   {
+    if constexpr (BY_TERM)
+      {
+        using CL = CacheLayout<DIM, G, TENS>;
+        return tangent_values_by_term<G>(pp, lin[CL::c], lin + CL::eta, v, vr);
+      }
     T g[G + 2][DIM], gr[G + 2][DIM];
 #pragma unroll
     for (int c = 0; c < G + 2; ++c)
@@ -416,8 +506,8 @@ namespace hps
     tangent_qp_rows<DIM, G, TENS, true, false>(pp, lin, v, g, vr, gr);
   }
 
-  template <int DIM, int G, bool TENS, typename T>
-  __device__ __forceinline__ void tangent_grad_c(const PhysParams &pp, const T *lin,
+  template <int DIM, int G, bool TENS, typename T, typename PP>
+  __device__ __forceinline__ void tangent_grad_c(const PP &pp, const T *lin,
                                                  const T *v, const T *g0, const T *g1,
                                                  T *out, const T *qsum = nullptr)
   {
@@ -443,8 +533,8 @@ namespace hps
   // residual QP operator: SinteringOperatorGenericResidualQuad::operator()
   // S/operator_sintering_generic.h:254-308; hist[] = sum_k w_k old_k at q
   // ------------------------------------------------------------------
-  template <int DIM, int G, bool TENS, int WTD, typename T>
-  __device__ __forceinline__ void residual_qp(const PhysParams &pp,
+  template <int DIM, int G, bool TENS, int WTD, typename T, typename PP>
+  __device__ __forceinline__ void residual_qp(const PP &pp,
                                               const T          *v,
                                               const T (*g)[DIM],
                                               const T          *hist,
@@ -478,17 +568,14 @@ namespace hps
     vr[0] = v0;
     if constexpr (!TENS)
       {
-        // MobilityScalar::apply_M, S/mobility.h:441-472
-        T etaijSum = T(0.0);
+        T sum = G > 0 ? etas[0] : T(0.0), pairs = T(0.0);
 #pragma unroll
-        for (int i = 0; i < G; ++i)
-#pragma unroll
-          for (int j = 0; j < i; ++j)
-            etaijSum += etas[i] * etas[j];
-        const T phi = phi_clamped(c);
-        const T M   = Mvol * phi + Mvap * (T(1.0) - phi) +
-                    Msurf * T(4.0) * c * c * (T(1.0) - c) * (T(1.0) - c) +
-                    (T(2.0) * Mgb) * etaijSum;
+        for (int i = 1; i < G; ++i)
+          {
+            pairs += etas[i] * sum;
+            sum += etas[i];
+          }
+        const T M = scalar_mobility(pp, c, c * (T(1.0) - c), pairs);
 #pragma unroll
         for (int d = 0; d < DIM; ++d)
           gr[0][d] = M * g[1][d];
@@ -539,8 +626,8 @@ namespace hps
       }
 
     // 2) mu row
-    const T df_dc = A * (c * c) * (T(2.0) * c - T(2.0)) +
-                    T(2.0) * A * c * ((-c + T(1.0)) * (-c + T(1.0))) +
+    // f_c = 2 A c (1 - c) (1 - 2 c) + B (2 c - 6 S2 + 4 S3)
+    const T df_dc = pp_A2<T>(pp) * (c * (T(1.0) - c)) * (T(1.0) - T(2.0) * c) +
                     B * (T(2.0) * c - T(6.0) * S2 + T(4.0) * S3);
     vr[1] = T(pp.w_alg) * v[1] - df_dc;
     const T kc = -T(pp.kappa_c);
@@ -554,7 +641,7 @@ namespace hps
     for (int i = 0; i < G; ++i)
       {
         const T e  = etas[i];
-        T       r  = L * (e * (B * T(12.0)) * (e * (T(1.0) * c - T(2.0)) + (-c + T(1.0)) + S2));
+        T       r  = (pp_BL12<T>(pp) * e) * (e * (c - T(2.0)) + ((T(1.0) - c) + S2));
         if constexpr (WTD >= 1)
           r += v[2 + i] * T(pp.w0);
         if constexpr (WTD == 2)
@@ -566,8 +653,8 @@ namespace hps
       }
   }
   // residual rows that need the state's values only (all rows' values)
-  template <int DIM, int G, bool TENS, int WTD, typename T>
-  __device__ __forceinline__ void residual_values(const PhysParams &pp, const T *v,
+  template <int DIM, int G, bool TENS, int WTD, typename T, typename PP>
+  __device__ __forceinline__ void residual_values(const PP &pp, const T *v,
                                                   const T *hist, T *vr)
   {
     T g[G + 2][DIM], gr[G + 2][DIM];
@@ -585,8 +672,8 @@ namespace hps
   // grain's pairs at a time: unrolled over all pairs at once, the divisions
   // of 45 pairs (10 order parameters) are in flight together and the
   // allocation needs 512 registers.
-  template <int DIM, int G, typename T>
-  __device__ __forceinline__ void residual_grad_c_tens(const PhysParams &pp, const T *v,
+  template <int DIM, int G, typename T, typename PP>
+  __device__ __forceinline__ void residual_grad_c_tens(const PP &pp, const T *v,
                                                        const T *gc, const T *gmu,
                                                        const T (*leg)[DIM], T *out)
   {
@@ -642,22 +729,20 @@ namespace hps
 
   // gradient row of c of the residual for scalar mobility: M(c, eta) grad mu
   // (MobilityScalar::apply_M, S/mobility.h:441-472)
-  template <int DIM, int G, typename T>
-  __device__ __forceinline__ void residual_grad_c_scalar(const PhysParams &pp, const T *v,
+  template <int DIM, int G, typename T, typename PP>
+  __device__ __forceinline__ void residual_grad_c_scalar(const PP &pp, const T *v,
                                                          const T *g1, T *out)
   {
     const T  c    = v[0];
     const T *etas = v + 2;
-    T        etaijSum = T(0.0);
+    T        sum = G > 0 ? etas[0] : T(0.0), pairs = T(0.0);
 #pragma unroll
-    for (int i = 0; i < G; ++i)
-#pragma unroll
-      for (int j = 0; j < i; ++j)
-        etaijSum += etas[i] * etas[j];
-    const T phi = phi_clamped(c);
-    const T M   = T(pp.Mvol) * phi + T(pp.Mvap) * (T(1.0) - phi) +
-                T(pp.Msurf) * T(4.0) * c * c * (T(1.0) - c) * (T(1.0) - c) +
-                (T(2.0) * T(pp.Mgb)) * etaijSum;
+    for (int i = 1; i < G; ++i)
+      {
+        pairs += etas[i] * sum;
+        sum += etas[i];
+      }
+    const T M = scalar_mobility(pp, c, c * (T(1.0) - c), pairs);
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
       out[d] = M * g1[d];
