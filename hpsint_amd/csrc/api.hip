@@ -905,9 +905,9 @@ static int precond_update(hps_operator op, int kind, bool fp32)
           HPS_HIP(hipMalloc(&op->inv_diag32, n * sizeof(float)));
         }
       if (op->q2 && fp32)
-        op->q2->probe32(q2_params(op), op->cache32, op->inv_diag32, -1, nc, 1, 0, op->stream);
+        op->q2->diag32(q2_params(op), op->cache32, op->inv_diag32, op->stream);
       else if (op->q2)
-        op->q2->probe(q2_params(op), op->cache64, op->diag, -1, nc, 1, 0, op->stream);
+        op->q2->diag(q2_params(op), op->cache64, op->diag, op->stream);
       else if (fp32)
         (op->cut_active ? op->ops->probe32_cut : op->ops->probe32)(
           op->kp, op->n_tiles, op->cache32, op->inv_diag32, (float *)op->part, -1, nc, 1, 0,
@@ -947,21 +947,20 @@ static int precond_update(hps_operator op, int kind, bool fp32)
         }
       // the assembled blocks are stored per node column by column
       // (blocks[node][column][row]): a block column is a contiguous run
-      if (op->q2) // all block columns in one pass over the cache
+      // Q2 (fe_q2_blocks.hpp) and Q1 in 3D with scalar mobility
+      // (fe_q1_blocks.hpp): every column from one pass, in FP64 from either
+      // cache; otherwise column by column
+      const bool one_pass = op->q2 || (op->dim == 3 && !op->tens && !op->cut_active &&
+                                       op->ops->tx == hps::TX3 && op->ops->ty == hps::TY3);
+      if (op->q2)
         {
           if (fp32)
-            op->q2->probe32(q2_params(op), op->cache32, op->inv_blocks32, -2, nc * nc, 1, 0,
-                            op->stream);
+            op->q2->blocks32(q2_params(op), op->cache32, op->blocks, op->stream);
           else
-            op->q2->probe(q2_params(op), op->cache64, op->blocks, -2, nc * nc, 1, 0,
-                          op->stream);
+            op->q2->blocks(q2_params(op), op->cache64, op->blocks, op->stream);
           HPS_LAUNCHED();
         }
-      // 3D scalar mobility: every column from one pass (fe_q1_blocks.hpp);
-      // otherwise column by column
-      const bool one_pass = !op->q2 && op->dim == 3 && !op->tens && !op->cut_active &&
-                            op->ops->tx == hps::TX3 && op->ops->ty == hps::TY3;
-      if (one_pass)
+      else if (one_pass)
         {
           if (!(fp32 ? hps::node_blocks_d3(op->n_grains, op->kp, op->cache32, op->blocks,
                                            op->stream) :
@@ -971,7 +970,7 @@ static int precond_update(hps_operator op, int kind, bool fp32)
                         "node-block Jacobi not built for this n_components");
           HPS_LAUNCHED();
         }
-      for (int j = 0; j < nc && !op->q2 && !one_pass; ++j)
+      for (int j = 0; j < nc && !one_pass; ++j)
         {
           if (fp32)
             (op->cut_active ? op->ops->probe32_cut : op->ops->probe32)(

@@ -1286,38 +1286,22 @@ namespace hps
       }
   }
 
-  // --------------------------------- diagonal / block column by probing
-  // For every local node j of the cell and input component b (all b for the
-  // diagonal, b = column for a block column) the cell's contribution to row
-  // (j, a) of the tangent, a = b for the diagonal and every a for a block
-  // column: sum_q JxW [phi_j (V_a) + grad phi_j . (G_a)] with (V, G) the
-  // quadrature operator applied to the increment e_b phi_j.  The operator is
-  // linear in (value, gradient) of the increment, so it is evaluated once
-  // per direction m of (value, d/dx, ...) with a unit input, and the node
-  // sums over the Gauss points run through LDS.  The result goes to
-  // dst[node * os + a * ocs + oo].
-  // ------------------------------------------------ diagonal / node blocks
-  // Node block B[j][a][b] = sum_q JxW psi_j,m'(q) M_{a m', b m}(q) psi_j,m(q)
+  // ------------------------------------------------------------ diagonal
+  // Entry (node j, component a) of the tangent's diagonal:
+  //   sum_q JxW psi_j,m'(q) M_{a m', a m}(q) psi_j,m(q)
   // (psi_j,0 = phi_j, psi_j,d+1 = d phi_j / dx_d; M: the quadrature-point
-  // tangent from input (component b, value or gradient d) to output
-  // (component a, value or gradient d')).  M is sparse: value rows read
-  // values only; the c gradient row reads the values and the gradients of
-  // c and mu; the mu and eta_i gradient rows are -kappa_c grad c and
-  // L kappa_p grad eta_i.  Each nonzero term is a tensor product of 1D
-  // weights w_q f(x_q) g(x_q) with f, g in {s_j, s_j'/h} per direction, so
-  // the q-sum is three sum-factorisation passes over the field M(q); terms
-  // with the same 1D weights share a field.  Rows (NR = n_c + 12):
-  //   r < n_c        phi phi           M_{r 0, b 0}          -> B[.][r][b]
-  //   n_c + d        phi' phi (dir d)  M_{0 d+1, b 0}        -> B[.][0][b]
-  //   n_c + 3 + d    phi' phi' (d, d)  M_{0 d+1, b d+1}      -> B[.][0][b]
-  //   n_c + 6 + p    phi' phi' (d, e)  M_{0 d+1, b e+1} + M_{0 e+1, b d+1}
-  //   n_c + 9 + d    phi' phi' (d, d)  -kappa_c (b = 0) -> B[.][1][0],
-  //                                    L kappa_p (b >= 2) -> B[.][b][b]
-  // The diagonal (column < 0) uses the same rows with the mass field of
-  // row b taken from input b, the c-row fields from input c, and the
-  // stiffness rows with field 1 scaled by L kappa_p for every b >= 2.
+  // tangent from input (component a, value or gradient d) to output
+  // (component a, value or gradient d')).  Each nonzero term is a tensor
+  // product of 1D weights w_q f(x_q) g(x_q) with f, g in {s_j, s_j'/h} per
+  // direction, so the q-sum is three sum-factorisation passes over the field
+  // M(q); terms with the same 1D weights share a field.  Rows (NR = n_c + 12):
+  //   r < n_c        phi phi           M_{r 0, r 0}          -> row r
+  //   n_c + d        phi' phi (dir d)  M_{0 d+1, 0 0}        -> row 0
+  //   n_c + 3 + d    phi' phi' (d, d)  M_{0 d+1, 0 d+1}      -> row 0
+  //   n_c + 6 + p    phi' phi' (d, e)  M_{0 d+1, 0 e+1} + M_{0 e+1, 0 d+1}
+  //   n_c + 9 + d    phi' phi' (d, d)  1, times L kappa_p    -> rows >= 2
   template <int DIM>
-  struct Q2ProbeRows
+  struct Q2DiagRows
   {
     // 1D weight type of row r along direction d: 0 phi phi, 1 phi' phi,
     // 2 phi' phi'
@@ -1339,204 +1323,131 @@ namespace hps
 
   template <int DIM, int G, bool TENS, typename T>
   __global__ void __launch_bounds__(64)
-    q2_probe(const Q2Params kp, const T *__restrict__ cache, T *__restrict__ dst, int column,
-             int os, int ocs, int oo)
+    q2_diag(const Q2Params kp, const T *__restrict__ cache, T *__restrict__ dst)
   {
     using CL         = CacheLayout<DIM, G, TENS>;
     constexpr int NC = G + 2;
     constexpr int NF = CL::n_fields;
     constexpr int NR = NC + 12;
     using LN         = Q2Lane<DIM>;
-    using RW         = Q2ProbeRows<DIM>;
+    using RW         = Q2DiagRows<DIM>;
 
     __shared__ T A[NR * 64];
     __shared__ T B[NR * 64];
 
     const LN  L(kp);
-    const int l    = L.l;
-    const T   kc   = -T(kp.pp.kappa_c);
-    const T   lkp  = T(kp.pp.L) * T(kp.pp.kappa_p);
+    const int l   = L.l;
+    const T   lkp = T(kp.pp.L) * T(kp.pp.kappa_p);
 
-    // entries of block column b (b < 0: the diagonal) of this lane's node,
-    // left in A[a * 64 + lane]
-    auto column_entries = [&](const int b) {
-      // 1) fields of the rows at this lane's Gauss point, into A
-      {
-        // (read again for every column, from the caches: the opaque offset
-        // keeps the loads inside the column loop, so the fields are not
-        // held in registers across it)
-        int off = 0;
-        asm volatile("" : "+v"(off));
-        T        lin[NF];
-        const T *cl = cache + ((kp.wg_base + blockIdx.x) * NF) * LN::LP + l + off;
+    // 1) fields of the rows at this lane's Gauss point, into A
+    {
+      T        lin[NF];
+      const T *cl = cache + ((kp.wg_base + blockIdx.x) * NF) * LN::LP + l;
 #pragma unroll
-        for (int f = 0; f < NF; ++f)
-          lin[f] = L.valid ? cl[f * LN::LP] : T(0);
-        const T zero[3] = {T(0), T(0), T(0)};
-        // c-row gradient outputs for the inputs of component cb: value (m = 0)
-        // and gradient d (m = d + 1)
-        auto c_rows = [&](int cb) {
-          T v[NC];
+      for (int f = 0; f < NF; ++f)
+        lin[f] = L.valid ? cl[f * LN::LP] : T(0);
+      const T zero[3] = {T(0), T(0), T(0)};
+#pragma unroll 1
+      for (int cb = 0; cb < NC; ++cb)
+        {
+          T v[NC], vr[NC];
 #pragma unroll
           for (int c = 0; c < NC; ++c)
             v[c] = c == cb ? T(1) : T(0);
-          T gm[DIM + 1][DIM];
-          tangent_grad_c<DIM, G, TENS>(kp.pp, lin, v, zero, zero, gm[0]);
+          tangent_values<DIM, G, TENS>(kp.pp, lin, v, vr);
+          T x = T(0);
 #pragma unroll
           for (int c = 0; c < NC; ++c)
-            v[c] = T(0);
+            if (c == cb)
+              x = vr[c];
+          A[cb * 64 + l] = x;
+        }
+      // c-row gradient outputs for the value of c (m = 0) and its gradient d
+      // (m = d + 1)
+      T v[NC];
 #pragma unroll
-          for (int d = 0; d < DIM; ++d)
-            {
-              T u[3] = {T(0), T(0), T(0)};
-              u[d]   = T(1);
-              if (cb <= 1)
-                tangent_grad_c<DIM, G, TENS>(kp.pp, lin, v, cb == 0 ? u : zero,
-                                             cb == 1 ? u : zero, gm[d + 1]);
-              else
+      for (int c = 0; c < NC; ++c)
+        v[c] = c == 0 ? T(1) : T(0);
+      T gm[DIM + 1][DIM];
+      tangent_grad_c<DIM, G, TENS>(kp.pp, lin, v, zero, zero, gm[0]);
+      v[0] = T(0);
 #pragma unroll
-                for (int e = 0; e < DIM; ++e)
-                  gm[d + 1][e] = T(0);
-            }
+      for (int d = 0; d < DIM; ++d)
+        {
+          T u[3] = {T(0), T(0), T(0)};
+          u[d]   = T(1);
+          tangent_grad_c<DIM, G, TENS>(kp.pp, lin, v, u, zero, gm[d + 1]);
+        }
 #pragma unroll
-          for (int d = 0; d < 3; ++d)
-            {
-              A[(NC + d) * 64 + l]     = d < DIM ? gm[0][d] : T(0);
-              A[(NC + 3 + d) * 64 + l] = d < DIM ? gm[d + 1][d] : T(0);
-            }
-          // pairs (0,1), (0,2), (1,2)
-          A[(NC + 6) * 64 + l] = gm[2][0] + gm[1][1];
-          A[(NC + 7) * 64 + l] = DIM == 3 ? gm[3 % (DIM + 1)][0] + gm[1][2 % DIM] : T(0);
-          A[(NC + 8) * 64 + l] = DIM == 3 ? gm[3 % (DIM + 1)][1] + gm[2][2 % DIM] : T(0);
-        };
-        if (b >= 0)
-          {
-            T v[NC], vr[NC];
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-              v[c] = c == b ? T(1) : T(0);
-            tangent_values<DIM, G, TENS>(kp.pp, lin, v, vr);
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-              A[c * 64 + l] = vr[c];
-            c_rows(b);
-            const T st = b == 0 ? kc : (b >= 2 ? lkp : T(0));
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-              A[(NC + 9 + d) * 64 + l] = d < DIM ? st : T(0);
-          }
-        else
-          {
-#pragma unroll 1
-            for (int cb = 0; cb < NC; ++cb)
-              {
-                T v[NC], vr[NC];
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-                  v[c] = c == cb ? T(1) : T(0);
-                tangent_values<DIM, G, TENS>(kp.pp, lin, v, vr);
-                T x = T(0);
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-                  if (c == cb)
-                    x = vr[c];
-                A[cb * 64 + l] = x;
-              }
-            c_rows(0);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-              A[(NC + 9 + d) * 64 + l] = d < DIM ? T(1) : T(0);
-          }
-      }
-      __syncthreads();
+      for (int d = 0; d < 3; ++d)
+        {
+          A[(NC + d) * 64 + l]     = d < DIM ? gm[0][d] : T(0);
+          A[(NC + 3 + d) * 64 + l] = d < DIM ? gm[d + 1][d] : T(0);
+          A[(NC + 9 + d) * 64 + l] = d < DIM ? T(1) : T(0);
+        }
+      // pairs (0,1), (0,2), (1,2)
+      A[(NC + 6) * 64 + l] = gm[2][0] + gm[1][1];
+      A[(NC + 7) * 64 + l] = DIM == 3 ? gm[3 % (DIM + 1)][0] + gm[1][2 % DIM] : T(0);
+      A[(NC + 8) * 64 + l] = DIM == 3 ? gm[3 % (DIM + 1)][1] + gm[2][2 % DIM] : T(0);
+    }
+    __syncthreads();
 
-      // 2) q -> node sums, one pass per direction over all rows
-      //    (A -> B -> A in 3D, the last pass into registers)
-      T res[NR];
-      {
-        T K[3][3]; // [type][q] for the current direction
-        auto coefs = [&](int d) {
-          T sc[3], ec[3];
-          q2_s_col(L.t[d], sc);
-          q2_e_col(L.t[d], ec);
+    // 2) q -> node sums, one pass per direction over all rows
+    //    (A -> B -> A in 3D, the last pass into registers)
+    T res[NR];
+    {
+      T K[3][3]; // [type][q] for the current direction
+      auto coefs = [&](int d) {
+        T sc[3], ec[3];
+        q2_s_col(L.t[d], sc);
+        q2_e_col(L.t[d], ec);
 #pragma unroll
-          for (int q = 0; q < 3; ++q)
-            {
-              const T w = q2_w<T>(q);
-              const T e = ec[q] * T(kp.inv_h[d]);
-              K[0][q]   = w * sc[q] * sc[q];
-              K[1][q]   = w * sc[q] * e;
-              K[2][q]   = w * e * e;
-            }
-        };
-        coefs(0);
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-          B[r * 64 + l] = q2_pass(A + r * 64, L.base(0), 1, K[RW::type(NC, r, 0)]);
-        __syncthreads();
-        coefs(1);
-        if constexpr (DIM == 3)
+        for (int q = 0; q < 3; ++q)
           {
-#pragma unroll
-            for (int r = 0; r < NR; ++r)
-              A[r * 64 + l] = q2_pass(B + r * 64, L.base(1), 3, K[RW::type(NC, r, 1)]);
-            __syncthreads();
-            coefs(2);
-#pragma unroll
-            for (int r = 0; r < NR; ++r)
-              res[r] = q2_pass(A + r * 64, L.base(2), 9, K[RW::type(NC, r, 2)]);
+            const T w = q2_w<T>(q);
+            const T e = ec[q] * T(kp.inv_h[d]);
+            K[0][q]   = w * sc[q] * sc[q];
+            K[1][q]   = w * sc[q] * e;
+            K[2][q]   = w * e * e;
           }
-        else
+      };
+      coefs(0);
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+        B[r * 64 + l] = q2_pass(A + r * 64, L.base(0), 1, K[RW::type(NC, r, 0)]);
+      __syncthreads();
+      coefs(1);
+      if constexpr (DIM == 3)
+        {
 #pragma unroll
           for (int r = 0; r < NR; ++r)
-            res[r] = q2_pass(B + r * 64, L.base(1), 3, K[RW::type(NC, r, 1)]);
-      }
-
-      // 3) rows to outputs
-      T acc[NC];
+            A[r * 64 + l] = q2_pass(B + r * 64, L.base(1), 3, K[RW::type(NC, r, 1)]);
+          __syncthreads();
+          coefs(2);
 #pragma unroll
-      for (int a = 0; a < NC; ++a)
-        acc[a] = res[a];
-      T c_sum = T(0), st_sum = T(0);
-#pragma unroll
-      for (int r = NC; r < NC + 9; ++r)
-        c_sum += res[r];
-#pragma unroll
-      for (int r = NC + 9; r < NR; ++r)
-        st_sum += res[r];
-      const T hp = T(kp.h_prod);
-      if (b >= 0)
-        {
-          acc[0] += c_sum;
-#pragma unroll
-          for (int a = 1; a < NC; ++a)
-            if (a == (b == 0 ? 1 : b) && b != 1)
-              acc[a] += st_sum;
+          for (int r = 0; r < NR; ++r)
+            res[r] = q2_pass(A + r * 64, L.base(2), 9, K[RW::type(NC, r, 2)]);
         }
       else
-        {
-          acc[0] += c_sum;
 #pragma unroll
-          for (int a = 2; a < NC; ++a)
-            acc[a] += lkp * st_sum;
-        }
-      __syncthreads();
+        for (int r = 0; r < NR; ++r)
+          res[r] = q2_pass(B + r * 64, L.base(1), 3, K[RW::type(NC, r, 1)]);
+    }
+
+    // 3) rows to entries
+    T c_sum = T(0), st_sum = T(0);
 #pragma unroll
-      for (int a = 0; a < NC; ++a)
-        A[a * 64 + l] = hp * acc[a];
-      __syncthreads();
-    };
-    // column -2: all block columns, column b of a node's block at
-    // dst + node * os + b * NC (the workgroup's cache stays in the caches
-    // between columns); otherwise the one column (or the diagonal) asked for
-    const bool all = column < -1;
-    const int  b0 = all ? 0 : column, b1 = all ? NC : column + 1;
-#pragma unroll 1
-    for (int b = b0; b < b1; ++b)
-      {
-        column_entries(b);
-        q2_scatter<DIM, NC, T>(kp, L, A, dst, os, all ? 1 : ocs, all ? b * NC : oo);
-        __syncthreads();
-      }
+    for (int r = NC; r < NC + 9; ++r)
+      c_sum += res[r];
+#pragma unroll
+    for (int r = NC + 9; r < NR; ++r)
+      st_sum += res[r];
+    const T hp = T(kp.h_prod);
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < NC; ++a)
+      A[a * 64 + l] = hp * (res[a] + (a == 0 ? c_sum : (a >= 2 ? lkp * st_sum : T(0))));
+    __syncthreads();
+    q2_scatter<DIM, NC, T>(kp, L, A, dst, NC, 1, 0);
   }
 } // namespace hps

@@ -6,6 +6,7 @@
 
 #include "fe_q1.hpp"
 #include "fe_q2.hpp"
+#include "fe_q2_blocks.hpp"
 
 namespace hps
 {
@@ -134,10 +135,11 @@ namespace hps
     void (*residual)(const Q2Params &, int wtd, const double *src, const double *o0,
                      const double *o1, const double *o2, double *dst, hipStream_t);
     void (*fill)(const Q2Params &, const double *lin, double *c64, float *c32, hipStream_t);
-    void (*probe)(const Q2Params &, const double *cache, double *dst, int column, int ostride,
-                  int ocstride, int ooffset, hipStream_t);
-    void (*probe32)(const Q2Params &, const float *cache, float *dst, int column, int ostride,
-                    int ocstride, int ooffset, hipStream_t);
+    // tangent diagonal, and node blocks (column by column)
+    void (*diag)(const Q2Params &, const double *cache, double *dst, hipStream_t);
+    void (*diag32)(const Q2Params &, const float *cache, float *dst, hipStream_t);
+    void (*blocks)(const Q2Params &, const double *cache, double *dst, hipStream_t);
+    void (*blocks32)(const Q2Params &, const float *cache, double *dst, hipStream_t);
   };
 
   // parameters of colour `col` (bit d = parity along d); wg: running count
@@ -252,24 +254,25 @@ namespace hps
         q2_fill<DIM, G, TENS><<<nb, 64, 0, s>>>(k, lin, c64, c32);
       });
     }
-    static void probe(const Q2Params &kp, const double *cache, double *dst, int column, int os,
-                      int ocs, int oo, hipStream_t s)
+    template <typename T>
+    static void diag(const Q2Params &kp, const T *cache, T *dst, hipStream_t s)
     {
       colours(kp, [&](const Q2Params &k, unsigned nb) {
-        q2_probe<DIM, G, TENS, double><<<nb, 64, 0, s>>>(k, cache, dst, column, os, ocs, oo);
+        q2_diag<DIM, G, TENS, T><<<nb, 64, 0, s>>>(k, cache, dst);
       });
     }
-    static void probe32(const Q2Params &kp, const float *cache, float *dst, int column, int os,
-                        int ocs, int oo, hipStream_t s)
+    template <typename T>
+    static void blocks(const Q2Params &kp, const T *cache, double *dst, hipStream_t s)
     {
       colours(kp, [&](const Q2Params &k, unsigned nb) {
-        q2_probe<DIM, G, TENS, float><<<nb, 64, 0, s>>>(k, cache, dst, column, os, ocs, oo);
+        q2_blocks<DIM, G, TENS, T><<<nb, 64, 0, s>>>(k, cache, dst);
       });
     }
     static Q2Table table()
     {
       return Q2Table{CacheLayout<DIM, G, TENS>::n_fields, CPW, &vmult64, &vmult32,
-                     &residual, &fill, &probe, &probe32};
+                     &residual, &fill, &diag<double>, &diag<float>,
+                     &blocks<double>, &blocks<float>};
     }
   };
 

@@ -440,8 +440,9 @@ namespace hps
   // ------------------------------------------------------------------
   // The value rows term by term (S/operator_sintering_generic.h:104-190),
   // with more operations than the collected form of tangent_qp_rows: the FP64
-  // Q2 tile march waits for memory, not for the VALU, and is scheduled better
-  // with them (96^3, 10 order parameters, tensorial: 3.42 against 3.58 ms).
+  // Q2 tile march waits for memory, not for the VALU.  The collected form gained
+  // it nothing, and with its derived products in the argument block it took
+  // 3.58 instead of 3.42 ms (96^3, 10 order parameters, tensorial).
   template <int G, typename T, typename PP>
   __device__ __forceinline__ void tangent_values_by_term(const PP &pp, T c, const T *etas,
                                                          const T *v, T *vr)

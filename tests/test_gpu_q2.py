@@ -206,3 +206,28 @@ def test_q2_fp32_preconditioner_assembly(dim, cells, G, tens):
     d = np.einsum("nii->ni", blocks_ref).ravel()
     _ffi.check(_ffi.lib().hps_precond_get_diagonal(op.handle, ctypes.c_void_p(inv.data_ptr())))
     assert rel_l2(host(inv), np.where(np.abs(d) > 1e-10, 1.0 / d, 1.0)) <= 1e-5
+
+
+@pytest.mark.parametrize("dim,cells,G,tens", [
+    (3, (1, 1, 1), 1, True), (3, (2, 3, 1), 1, False), (3, (3, 2, 3), 5, True),
+    (3, (2, 3, 2), 7, False), (3, (3, 3, 2), 10, True), (3, (2, 2, 3), 12, True),
+    (2, (1, 1), 1, True), (2, (8, 3), 6, False), (2, (5, 7), 12, True)])
+def test_q2_node_blocks_of_every_shape(dim, cells, G, tens):
+    """node blocks formed in one pass, odd and even block sizes, ragged colours:
+    FP64 to the tolerance of the other FP64 comparisons; from the FP32 cache
+    each block entry is a sum of 27 products of about 10 roundings each, half
+    an ulp (2^-24) apiece and of both signs: 60 of them, 4e-6, in the norm"""
+    import ctypes
+    from hpsint_amd import _ffi
+    op, p = make_pair(dim, cells, G, tens, w0=1000.0)
+    u = fields(p, 16)
+    ref = po.node_blocks(p, po.fill_qp(p, u))
+    op.fill_quadrature_point_values(dev(u))
+    got = host(op.node_blocks()).reshape(ref.shape)
+    assert rel_l2(got, ref) <= TOL64, rel_l2(got, ref)
+    P = Preconditioner(op, "InverseComponentBlockDiagonalMatrix")
+    P.do_update(fp32=True)
+    b = torch.empty(ref.size, dtype=torch.float64, device="cuda")
+    _ffi.check(_ffi.lib().hps_precond_get_blocks(op.handle, ctypes.c_void_p(b.data_ptr())))
+    got = host(b).reshape(ref.shape)
+    assert rel_l2(got, ref) <= 4e-6, rel_l2(got, ref)
