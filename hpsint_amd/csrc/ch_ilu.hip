@@ -32,8 +32,9 @@
 //   (mu, c):  JxW (-d2f/dc2 phi_m phi_k - kappa_c grad phi_m . grad phi_k)
 //   (mu, mu): JxW w_alg phi_m phi_k
 // (S/operator_sintering_generic.h:104-190 with MobilityScalar,
-// S/mobility.h:441-534), in 2^DIM cell-parity passes so that no two threads
-// add to one node's row.
+// S/mobility.h:441-534): in 3D by node planes, every row written once
+// (k_ch_assemble_z); in 2D and with tensorial mobility in 2^DIM cell-parity
+// passes so that no two threads add to one node's row.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -198,6 +199,305 @@ namespace hps
             ra[s4 + 1] += jxw * a1;
             ra[s4 + 2] += jxw * a2;
             ra[s4 + 3] += jxw * a3;
+          }
+      }
+  }
+
+  // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs
+  // on XCD b % 8).  The logical block returned here gives each XCD one
+  // contiguous range of the colour grid, so that the neighbour rows a stage
+  // gathers from the other colours are shared in that XCD's L2.  The map is
+  // a bijection of [0, gridDim.x): XCD x < r takes q + 1 blocks, the others
+  // q, with nb = 8 q + r.
+  __device__ __forceinline__ int xcd_block()
+  {
+    const int nb = (int)gridDim.x, b = (int)blockIdx.x;
+    const int q = nb >> 3, r = nb & 7, x = b & 7, k = b >> 3;
+    return x * q + (x < r ? x : r) + k;
+  }
+
+  // 3D, scalar mobility: every row entry formed in registers and written once.
+  // A workgroup completes the rows of 15 x 7 nodes (x, y) on the node planes
+  // z0 .. z0 + zn - 1, marching through the 16 x 8 cells around them layer by
+  // layer.  Lane (i, j) of a layer evaluates the coefficients of cell (i, j)
+  // at its 8 Gauss points into LDS: -JxW f''_cc, JxW M, JxW dM/dc grad mu_d /
+  // h_d.  It owns the node at that cell's lower corner, so the node's cells in
+  // the layer are those of lanes (i - kx, j - ky), in which it is corner
+  // (kx, ky, kz).  kz = 0 adds to the entries within its node plane (begun in
+  // the layer below) and forms those to the plane above; kz = 1 forms those to
+  // the plane below of the next node plane.  With all indices relative to
+  // corner k (bit set: the other side) one corner's sums are the same
+  // sum-factorised butterflies for every k but for the gradients' signs.
+  // (Adding each cell's element matrix to its rows, in 8 cell-parity passes,
+  // read and wrote a row 8 times.)
+  // Bound: FP64 VALU issue and the 864 bytes written per node; 129^3 nodes, 4
+  // order parameters: 1.06 ms (4.6 with the passes; the bytes take 0.6).
+  namespace cha
+  {
+    constexpr int WX = 16, WY = 8, OX = WX - 1, OY = WY - 1, NT = WX * WY;
+    constexpr double sa = 0.78867513459481288225457439025098;
+    constexpr double sb = 0.21132486540518711774542560974902;
+    // f (bit b of the index: direction b) <- along direction D:
+    // sum_q N_k N_m f: N_m = N_k, N_m the other
+    template <int D>
+    __device__ __forceinline__ void mass(double *f)
+    {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (!(i >> D & 1))
+          {
+            const double a = f[i], b = f[i | 1 << D];
+            f[i]           = sa * sa * a + sb * sb * b;
+            f[i | 1 << D]  = sa * sb * (a + b);
+          }
+    }
+    // sum_q N_m f
+    template <int D>
+    __device__ __forceinline__ void value(double *f)
+    {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (!(i >> D & 1))
+          {
+            const double a = f[i], b = f[i | 1 << D];
+            f[i]           = sa * a + sb * b;
+            f[i | 1 << D]  = sb * a + sa * b;
+          }
+    }
+    // sum_q of both, in the entry of N_m = N_k, its negative in the other
+    template <int D>
+    __device__ __forceinline__ void diff(double *f)
+    {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (!(i >> D & 1))
+          {
+            f[i] += f[i | 1 << D];
+            f[i | 1 << D] = -f[i];
+          }
+    }
+  } // namespace cha
+
+  __global__ void __launch_bounds__(cha::NT) __attribute__((amdgpu_waves_per_eu(2)))
+    k_ch_assemble_z(const ChParams cp, const double *__restrict__ cache, double *__restrict__ A,
+                    int zn)
+  {
+    using namespace cha;
+    constexpr int NFD = 5;
+    __shared__ double cf[NFD * 8][NT];
+
+    const int tid = (int)threadIdx.x, ci = tid & (WX - 1), cj = tid / WX;
+    const int nwx = (cp.nn[0] + OX - 1) / OX, nwy = (cp.nn[1] + OY - 1) / OY;
+    const int b   = xcd_block();
+    const int gx = (b % nwx) * OX - 1 + ci, gy = ((b / nwx) % nwy) * OY - 1 + cj;
+    const int z0 = (b / (nwx * nwy)) * zn, z1 = min(z0 + zn, cp.nn[2]);
+    const bool in_cell = gx >= 0 && gx < cp.nc[0] && gy >= 0 && gy < cp.nc[1];
+    const bool own     = ci > 0 && cj > 0 && gx < cp.nn[0] && gy < cp.nn[1];
+    // the cell's place in the cache (as k_ch_assemble)
+    const int64_t ntl   = cp.nt_lanes;
+    const int64_t tile0 = in_cell ? (gx / cp.tx) + (int64_t)cp.nt[0] * (gy / cp.ty) : 0;
+    const int     lane0 = in_cell ? ((gy % cp.ty) * cp.tx + gx % cp.tx) << 3 : 0;
+
+    double mid[9][3];
+#pragma unroll
+    for (int s = 0; s < 9; ++s)
+      mid[s][0] = mid[s][1] = mid[s][2] = 0.0;
+
+    // corner (KX, KY, KZ) of the cell of lane (ci - KX, cj - KY): added to
+    // same (node plane of the lane's node) and to other (the plane across)
+    auto corner = [&](auto K, double (*same)[3], double (*other)[3]) {
+      constexpr int k = K, kx = k & 1, ky = (k >> 1) & 1;
+      // (lanes without a node read their own cell's values)
+      const int src = own ? tid - kx - WX * ky : tid;
+      auto      at  = [&](int f, int q) { return cf[f * 8 + (q ^ k)][src]; };
+      // (one field's reads at a time: hoisted, the reads of all corners would
+      // spill)
+      auto      hold = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto      add = [&](int a, const double *f) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+          {
+            const int dx = (m & 1) ? (kx ? -1 : 1) : 0, dy = (m & 2) ? (ky ? -1 : 1) : 0;
+            double   &t  = ((m & 4) ? other : same)[(dx + 1) + 3 * (dy + 1)][a];
+            t += f[m];
+            // (the compiler otherwise moves the sums into the conditional
+            // store, with all of their inputs alive)
+            asm volatile("" : "+v"(t));
+          }
+      };
+      double f[8];
+      hold();
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        f[q] = at(0, q);
+      mass<0>(f);
+      mass<1>(f);
+      mass<2>(f);
+      add(2, f);
+      {
+        double M[8], r[8];
+        hold();
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          M[q] = at(1, q);
+        auto dir = [&](auto D) {
+          constexpr int d = D, e = (d + 1) % 3, g = (d + 2) % 3;
+          const double  h2 = cp.inv_h[d] * cp.inv_h[d];
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            f[q] = M[q];
+          diff<d>(f);
+          mass<e>(f);
+          mass<g>(f);
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            r[q] = d == 0 ? h2 * f[q] : r[q] + h2 * f[q];
+        };
+        dir(std::integral_constant<int, 0>{});
+        dir(std::integral_constant<int, 1>{});
+        dir(std::integral_constant<int, 2>{});
+        add(1, r);
+      }
+      auto dir = [&](auto D) {
+        constexpr int    d = D, e = (d + 1) % 3, g = (d + 2) % 3;
+        constexpr double s = (k >> d & 1) ? 1.0 : -1.0;
+        hold();
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+          f[q] = s * at(2 + d, q);
+        value<d>(f);
+        mass<e>(f);
+        mass<g>(f);
+        add(0, f);
+      };
+      dir(std::integral_constant<int, 0>{});
+      dir(std::integral_constant<int, 1>{});
+      dir(std::integral_constant<int, 2>{});
+    };
+
+    // sum over the shared cells of the products of the 1D shape functions of
+    // two nodes at distance o along d, and of their derivatives times h^2
+    auto m1 = [&](int d, int x, int o) {
+      const double cells = o ? ((o < 0 ? x > 0 : x < cp.nc[d]) ? 1.0 : 0.0) :
+                               (x > 0 ? 1.0 : 0.0) + (x < cp.nc[d] ? 1.0 : 0.0);
+      return cells * (o ? 2.0 * sa * sb : sa * sa + sb * sb);
+    };
+    auto k1 = [&](int d, int x, int o) {
+      const double cells = o ? ((o < 0 ? x > 0 : x < cp.nc[d]) ? 1.0 : 0.0) :
+                               (x > 0 ? 1.0 : 0.0) + (x < cp.nc[d] ? 1.0 : 0.0);
+      return (o ? -2.0 : 2.0) * cells * (cp.inv_h[d] * cp.inv_h[d]);
+    };
+    // the 9 entries of the lane's node on plane z to plane z + dz
+    auto store = [&](int z, int dz, const double (*acc)[3]) {
+      if (!own)
+        return;
+      // (through an empty asm statement: the node's factors below are formed
+      // here, not held across the march)
+      int x = gx, y = gy;
+      asm volatile("" : "+v"(x), "+v"(y));
+      const int     zc = (z & 1) << 2;
+      const bool    xo = x & 1, yo = y & 1;
+      auto          pick = [&](auto *v) {
+        const auto a = xo ? v[zc | 1] : v[zc], c = xo ? v[zc | 3] : v[zc | 2];
+        return yo ? c : a;
+      };
+      const int64_t cnt = pick(cp.cnt);
+      const int64_t ic  = (x >> 1) + (int64_t)pick(cp.mx) * ((y >> 1) + (int64_t)pick(cp.my) * (z >> 1));
+      double4      *r   = reinterpret_cast<double4 *>(A + pick(cp.off)) + ic + 9 * (dz + 1) * cnt;
+      const double  mz = cp.jxw * m1(2, z, dz), kz = cp.jxw * k1(2, z, dz);
+#pragma unroll
+      for (int s = 0; s < 9; ++s)
+        {
+          const int    ox = s % 3 - 1, oy = s / 3 - 1;
+          const double mx = m1(0, x, ox), my = m1(1, y, oy);
+          const double mm = mx * my * mz;
+          const double kk = k1(0, x, ox) * my * mz + mx * k1(1, y, oy) * mz + mx * my * kz;
+          r[s * cnt]      = double4{acc[s][0] + cp.pp.w0 * mm, acc[s][1],
+                               acc[s][2] - cp.pp.kappa_c * kk, cp.pp.w_alg * mm};
+        }
+    };
+
+    for (int L = z0 - 1; L < z1; ++L)
+      {
+        // coefficients of the lane's cell in layer L (zero outside the mesh)
+        const bool    in = in_cell && L >= 0 && L < cp.nc[2];
+        const double *cl = cache + lane0;
+        if (in)
+          cl += ((tile0 + (int64_t)cp.nt[0] * cp.nt[1] * (L / cp.tz)) * cp.tz + L % cp.tz) *
+                cp.nf * ntl;
+        __syncthreads();
+#pragma unroll 2
+        for (int h = 0; h < 4; ++h)
+          {
+            auto   load = [&](int f) {
+              return in ? reinterpret_cast<const double2 *>(cl + f * ntl)[h] : double2{0.0, 0.0};
+            };
+            const double2 c2 = load(0);
+            double2       mu[3], sum{0.0, 0.0}, pairs{0.0, 0.0};
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+              mu[d] = load(1 + cp.G + d);
+#pragma unroll 4
+            for (int g = 0; g < cp.G; ++g)
+              {
+                const double2 e = load(1 + g);
+                pairs.x += e.x * sum.x;
+                pairs.y += e.y * sum.y;
+                sum.x += e.x;
+                sum.y += e.y;
+              }
+            const double j = in ? cp.jxw : 0.0;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+              {
+                const int    q   = 2 * h + t;
+                const double c   = t ? c2.y : c2.x;
+                const double phi = dmin(1.0, dmax(0.0, c * c * c * (10.0 - 15.0 * c + 6.0 * c * c)));
+                const double p   = c * (1.0 - c);
+                const double M   = cp.pp.Mvol * phi + cp.pp.Mvap * (1.0 - phi) +
+                                 cp.pp.Msurf * 4.0 * (p * p) +
+                                 (2.0 * cp.pp.Mgb) * (t ? pairs.y : pairs.x);
+                const double dM = 30.0 * (cp.pp.Mvol - cp.pp.Mvap) * (p * p) +
+                                  cp.pp.Msurf * 8.0 * p * (1.0 - 2.0 * c);
+                const double d2 = 12.0 * cp.pp.A * (c * (c - 1.0)) + 2.0 * (cp.pp.A + cp.pp.B);
+                cf[q][tid]      = -j * d2;
+                cf[8 + q][tid]  = j * M;
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                  cf[(2 + d) * 8 + q][tid] = j * dM * (t ? mu[d].y : mu[d].x) * cp.inv_h[d];
+              }
+          }
+        __syncthreads();
+        if (L >= z0)
+          {
+            double up[9][3];
+#pragma unroll
+            for (int s = 0; s < 9; ++s)
+              up[s][0] = up[s][1] = up[s][2] = 0.0;
+            corner(std::integral_constant<int, 0>{}, mid, up);
+            corner(std::integral_constant<int, 1>{}, mid, up);
+            corner(std::integral_constant<int, 2>{}, mid, up);
+            corner(std::integral_constant<int, 3>{}, mid, up);
+            store(L, 0, mid);
+            store(L, 1, up);
+          }
+        if (L + 1 < z1)
+          {
+            double down[9][3];
+#pragma unroll
+            for (int s = 0; s < 9; ++s)
+              {
+                mid[s][0] = mid[s][1] = mid[s][2] = 0.0;
+                down[s][0] = down[s][1] = down[s][2] = 0.0;
+              }
+            corner(std::integral_constant<int, 4>{}, mid, down);
+            corner(std::integral_constant<int, 5>{}, mid, down);
+            corner(std::integral_constant<int, 6>{}, mid, down);
+            corner(std::integral_constant<int, 7>{}, mid, down);
+            store(L + 1, -1, down);
           }
       }
   }
@@ -558,19 +858,6 @@ namespace hps
       }
   }
 
-  // Workgroups are dispatched to the 8 XCDs round-robin (workgroup b runs
-  // on XCD b % 8).  The logical block returned here gives each XCD one
-  // contiguous range of the colour grid, so that the neighbour rows a stage
-  // gathers from the other colours are shared in that XCD's L2.  The map is
-  // a bijection of [0, gridDim.x): XCD x < r takes q + 1 blocks, the others
-  // q, with nb = 8 q + r.
-  __device__ __forceinline__ int xcd_block()
-  {
-    const int nb = (int)gridDim.x, b = (int)blockIdx.x;
-    const int q = nb >> 3, r = nb & 7, x = b & 7, k = b >> 3;
-    return x * q + (x < r ? x : r) + k;
-  }
-
   template <int DIM, int COL>
   __global__ void __launch_bounds__(256)
     k_ch_factor(const ChParams cp, double *__restrict__ A, float *__restrict__ A32)
@@ -830,6 +1117,19 @@ namespace hps
 
   void ch_assemble(const ChParams &cp, const double *cache, double *A, hipStream_t s)
   {
+    if (cp.dim == 3 && !cp.tens)
+      {
+        // planes per march: as the node blocks, enough marches for four rounds
+        // of the 768 workgroups that run at once while the mesh allows it
+        const int64_t cols = (int64_t)((cp.nn[0] + cha::OX - 1) / cha::OX) *
+                             ((cp.nn[1] + cha::OY - 1) / cha::OY);
+        int64_t zn = cols * cp.nn[2] / 3072;
+        zn         = zn < 4 ? 4 : (zn > 32 ? 32 : zn);
+        const int64_t chunks = (cp.nn[2] + zn - 1) / zn;
+        zn                   = (cp.nn[2] + chunks - 1) / chunks;
+        k_ch_assemble_z<<<(unsigned)(cols * chunks), cha::NT, 0, s>>>(cp, cache, A, (int)zn);
+        return;
+      }
     const int64_t nA = cp.n_nodes * (cp.dim == 3 ? 27 : 9) * 4;
     (void)hipMemsetAsync(A, 0, nA * sizeof(double), s);
     for (int par = 0; par < (1 << cp.dim); ++par)
@@ -842,8 +1142,6 @@ namespace hps
           continue;
         if (cp.tens)
           ch_assemble_tens(cp, par, n, cache, A, s);
-        else if (cp.dim == 3)
-          k_ch_assemble<3><<<blocks_for(n), 256, 0, s>>>(cp, par, cache, A);
         else
           k_ch_assemble<2><<<blocks_for(n), 256, 0, s>>>(cp, par, cache, A);
       }

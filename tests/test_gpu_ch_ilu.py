@@ -72,6 +72,15 @@ def test_ch_ilu_random_fields(cells, G):
     check(mesh, G, u.ravel())
 
 
+@pytest.mark.parametrize("cells,G", [((1, 1, 1), 1), ((14, 6, 3), 2), ((15, 7, 4), 3),
+                                     ((16, 8, 2), 5), ((30, 1, 1), 8), ((2, 15, 33), 1),
+                                     ((5, 3, 4), 12)])
+def test_ch_ilu_at_the_edges_of_the_assembly_tiles(cells, G):
+    """3D scalar assembly: 15 x 7 nodes and a run of planes per workgroup; mesh
+    sizes one node below, at and above a tile, one cell thick, several runs"""
+    test_ch_ilu_random_fields(cells, G)
+
+
 @pytest.mark.parametrize("cells,G", [((9, 5, 7), 2), ((6, 7, 5), 4), ((13, 9), 3),
                                      ((5, 6, 4), 7), ((4, 5, 3), 12)])
 def test_ch_ilu_tensorial_mobility(cells, G):
