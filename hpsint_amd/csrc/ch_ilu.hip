@@ -765,26 +765,43 @@ namespace hps
     }
   };
 
-  // row (i, AR) (AR = 0: c, 1: mu) of the nodes of colour COL, held in
-  // registers: R[s] = the entries (AR, c) and (AR, mu) of stencil entry s.
+  // the value of the lane pair's even lane
+  __device__ __forceinline__ double even_lane(double x)
+  {
+    constexpr int from = 0xA0; // quad_perm [0, 0, 2, 2]
+    const int     lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), from, 0xf, 0xf, true);
+    const int     hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), from, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+  }
+
+  // rows (i, c) and (i, mu) of the nodes of colour COL, one lane each (ar = 0:
+  // c, 1: mu; the lanes of a pair read the same neighbour rows and write one
+  // run), held in registers: R[s] = the entries (ar, c) and (ar, mu) of stencil
+  // entry s.
   // IKJ order: the lower entries (j, b) in increasing column order -- the
   // neighbours j of lower colours by (colour, index), c before mu, and for
-  // the mu row finally (i, c) -- each eliminated with the already final row
-  // (j, b): l = a / u_(j,b),(j,b); a_(i,AR),(k,e) -= l u_(j,b),(k,e) for
+  // the mu row finally (i, c), from the other lane -- each eliminated with the
+  // already final row
+  // (j, b): l = a / u_(j,b),(j,b); a_(i,ar),(k,e) -= l u_(j,b),(k,e) for
   // the (k, e) after (j, b) in row (j, b) that are in the pattern of row
-  // (i, AR): (j, mu) when b = c, and the neighbours k of j of a higher
+  // (i, ar): (j, mu) when b = c, and the neighbours k of j of a higher
   // colour than j's that are neighbours of i (or i itself).  Entries of
   // neighbours outside the domain are zero in the assembled block and stay
   // zero.  The final row is written in FP64 and FP32.
-  template <int DIM, int COL, int AR>
+  // Bound: latency of the neighbour rows at 2 waves per SIMD, and the rows of
+  // the lower colours read again by each stage.  129^3 nodes: 2.7 ms for the 8
+  // stages; with one lane per node, which formed row c and then row mu, every
+  // neighbour row was read twice, one after the other: 4.9 ms.
+  template <int DIM, int COL>
   __device__ __forceinline__ void ch_factor_row(const ChParams &cp, const ColourNode<DIM, COL> &n,
-                                                double *__restrict__ A, float *__restrict__ A32)
+                                                const int ar, double *__restrict__ A,
+                                                float *__restrict__ A32)
   {
     constexpr int                   S      = DIM == 3 ? 27 : 9;
     constexpr int                   center = (S - 1) / 2;
     constexpr FactorLists<DIM, COL> fl{};
     constexpr int px = COL & 1, py = (COL >> 1) & 1, pz = (COL >> 2) & 1;
-    double2      *Ai = reinterpret_cast<double2 *>(A + cp.off[COL]) + 2 * n.ic + AR;
+    double2      *Ai = reinterpret_cast<double2 *>(A + cp.off[COL]) + 2 * n.ic + ar;
     const int64_t st = 2 * cp.cnt[COL];  // double2 stride between stencil entries
     double        R[S][2];
 #pragma unroll
@@ -833,23 +850,27 @@ namespace hps
             R[v][1] -= l1 * uu.w;
           }
       }
-    if (AR == 1)
+    // the lower entry (i, c) of row (i, mu), with the final row (i, c) of the
+    // pair's even lane
+    const double cx = even_lane(R[center][0]), cy = even_lane(R[center][1]);
+    const double l  = R[center][0] / cx;
+    if (ar)
       {
-        // the lower entry (i, c) of row (i, mu), with the final row (i, c)
-        const double2 *Ac = Ai - 1;
-        const double2  cc = Ac[center * st];
-        const double   l  = R[center][0] / cc.x;
-        R[center][0]      = l;
-        R[center][1] -= l * cc.y;
+        R[center][0] = l;
+        R[center][1] -= l * cy;
+      }
 #pragma unroll
-        for (int t = 0; t < fl.n_upper; ++t)
+    for (int t = 0; t < fl.n_upper; ++t)
+      {
+        const int    u  = fl.upper[t];
+        const double ux = even_lane(R[u][0]), uy = even_lane(R[u][1]);
+        if (ar)
           {
-            const double2 cu = Ac[fl.upper[t] * st];
-            R[fl.upper[t]][0] -= l * cu.x;
-            R[fl.upper[t]][1] -= l * cu.y;
+            R[u][0] -= l * ux;
+            R[u][1] -= l * uy;
           }
       }
-    float2 *Ai32 = reinterpret_cast<float2 *>(A32 + cp.off[COL]) + 2 * n.ic + AR;
+    float2 *Ai32 = reinterpret_cast<float2 *>(A32 + cp.off[COL]) + 2 * n.ic + ar;
 #pragma unroll
     for (int s = 0; s < S; ++s)
       {
@@ -862,12 +883,11 @@ namespace hps
   __global__ void __launch_bounds__(256)
     k_ch_factor(const ChParams cp, double *__restrict__ A, float *__restrict__ A32)
   {
-    const int64_t ic = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
+    const int64_t ic = (int64_t)xcd_block() * 128 + (threadIdx.x >> 1);
     if (ic >= cp.cnt[COL])
       return;
     const ColourNode<DIM, COL> n(cp, ic);
-    ch_factor_row<DIM, COL, 0>(cp, n, A, A32);
-    ch_factor_row<DIM, COL, 1>(cp, n, A, A32);
+    ch_factor_row<DIM, COL>(cp, n, (int)threadIdx.x & 1, A, A32);
   }
 
   // ------------------------------------------------------------------ solves
@@ -1151,7 +1171,7 @@ namespace hps
   static void ch_factor_stages(std::integer_sequence<int, C...>, const ChParams &cp, double *A,
                                float *A32, hipStream_t s)
   {
-    ((cp.cnt[C] ? k_ch_factor<DIM, C><<<blocks_for(cp.cnt[C]), 256, 0, s>>>(cp, A, A32) : void()),
+    ((cp.cnt[C] ? k_ch_factor<DIM, C><<<blocks_for(2 * cp.cnt[C]), 256, 0, s>>>(cp, A, A32) : void()),
      ...);
   }
 
