@@ -1,0 +1,108 @@
+"""Reductions whose grid follows the vector's length, and the tile depth that
+follows the mesh, at the edges of their rules."""
+import ctypes
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from hpsint_amd import _ffi  # noqa: E402
+from hpsint_amd.operator import (CartesianMesh, FreeEnergyParams, MobilityParams,  # noqa: E402
+                                 SinteringOperatorGeneric)
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(x, dtype=torch.float64):
+    return torch.as_tensor(np.ascontiguousarray(x), dtype=dtype).cuda()
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.detach().cpu().numpy().astype(np.float64)
+
+
+# one block, one block and its neighbour, the last length of a growing grid,
+# the full grid with and without a remainder
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 1025, 2048 * 512, 2048 * 512 + 1, 3000001])
+@pytest.mark.parametrize("k", [1, 16, 17, 31])
+def test_reductions_at_the_edges_of_the_grid_rule(n, k):
+    """A sum of FP64 products: a thread adds at most n / 2^19 + 2 of them, then
+    17 levels of trees and rows follow, each rounding at most half an ulp
+    (2^-53) of the sum of magnitudes: 32 + n / 2^19 halves.  An update w -=
+    sum h_j V_j rounds once per product and once per sum: 2 k + 2 halves of the
+    storage type, relative to the magnitudes."""
+    mesh = CartesianMesh((2, 2, 2), (0, 0, 0), (2.0, 2.0, 2.0))
+    op = SinteringOperatorGeneric(mesh, 1)
+    h, L = op.handle, _ffi.lib()
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    rng = np.random.default_rng(n + k)
+    tol = (32 + n / 2**19) * 2.0**-53
+    r = ctypes.c_double()
+    hh = (ctypes.c_double * k)()
+    for dtype, npt, ulp, suf in ((torch.float64, np.float64, 2.0**-53, ""),
+                                 (torch.float32, np.float32, 2.0**-24, "_f32")):
+        V = rng.standard_normal((k, n)).astype(npt)
+        w = rng.standard_normal(n).astype(npt)
+        V64, w64 = V.astype(np.longdouble), w.astype(np.longdouble)
+        dV, dw = dev(V.ravel(), dtype), dev(w, dtype)
+        _ffi.check(getattr(L, "hps_norm2" + suf)(h, n, P(dw), ctypes.byref(r)))
+        ref = np.sqrt(np.sum(w64 * w64))
+        assert abs(r.value - ref) <= tol * ref
+        _ffi.check(getattr(L, "hps_multi_dot" + suf)(h, n, k, P(dV), P(dw), hh))
+        for j in range(k):
+            ref, mag = np.sum(V64[j] * w64), np.sum(np.abs(V64[j] * w64))
+            assert abs(hh[j] - ref) <= tol * mag, (j, hh[j], ref)
+        _ffi.check(getattr(L, "hps_multi_axpy_norm" + suf)(h, n, k, P(dV), hh, P(dw),
+                                                          ctypes.byref(r)))
+        c = np.array(list(hh), dtype=np.longdouble)
+        ref, mag = w64 - c @ V64, np.abs(w64) + np.abs(c) @ np.abs(V64)
+        got = host(dw)
+        assert np.all(np.abs(got - ref) <= (2 * k + 2) * ulp * mag)
+        nrm = np.sqrt(np.sum(got.astype(np.longdouble)**2))
+        # (n = 1: everything cancels and the norm is of rounding errors)
+        slack = tol * nrm + (2 * k + 2) * ulp * np.sqrt(np.sum(mag**2))
+        assert abs(r.value - nrm) <= slack
+
+
+@pytest.mark.parametrize("cells,G,tens", [
+    ((24, 24, 24), 4, False),   # fewest layers per tile
+    ((24, 24, 24), 5, False),   # fewest of five and more order parameters
+    ((64, 40, 33), 3, False),   # between
+    ((96, 96, 70), 2, False),   # unchanged
+    ((160, 81), 2, False), ((33, 500), 3, True), ((17, 9, 30), 3, True)])
+def test_tile_depth_of_small_meshes(monkeypatch, cells, G, tens):
+    """tangent, residual and diagonal with the depth chosen for the mesh against
+    16 layers.  Only the order in which the cells of a node are added differs:
+    8 (2D 4) cell sums, 8 roundings of half an ulp of values that may cancel to
+    about a tenth: 1e-14 in the norm"""
+    dim = len(cells)
+    mesh = CartesianMesh(cells, (0.0,) * dim, tuple(0.5 * c for c in cells))
+    nn = int(np.prod([c + 1 for c in cells]))
+    rng = np.random.default_rng(G)
+    u = rng.uniform(0, 1, size=(nn, G + 2))
+    src = rng.uniform(-1, 1, size=u.size)
+
+    def results():
+        op = SinteringOperatorGeneric(mesh, G, FreeEnergyParams(), MobilityParams(tensorial=tens))
+        op.set_time_weights(1000.0, (-1000.0,))
+        op.fill_quadrature_point_values(dev(u.ravel()))
+        out = []
+        for dtype in (torch.float64, torch.float32):
+            dst = op.initialize_dof_vector(dtype)
+            op.vmult(dst, dev(src, dtype))
+            out.append(host(dst))
+        dst = op.initialize_dof_vector()
+        op.evaluate_nonlinear_residual(dst, dev(u.ravel()), 2, old=[dev(0.9 * u.ravel())])
+        out.append(host(dst))
+        inv = op.initialize_dof_vector()
+        op.compute_inverse_diagonal(inv)
+        out.append(host(inv))
+        return out
+
+    got = results()
+    monkeypatch.setenv("HPSINT_AMD_TILE_M", "16")
+    ref = results()
+    for g, r, tol in zip(got, ref, (1e-14, 1e-14 * 2.0**29, 1e-14, 1e-14)):
+        assert np.linalg.norm(g - r) <= tol * np.linalg.norm(r)
