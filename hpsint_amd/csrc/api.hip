@@ -355,10 +355,11 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
       // one-lane-per-corner kernel
       const bool zc = prm->dim == 3 && !tens && ops->tx == hps::TX3 && ops->ty == hps::TY3 &&
                       env_int("HPSINT_AMD_ZCOL", 1) != 0;
-      op->zcol   = zc && G <= hps::ZCOL_MAX_G;
       op->zcol32 = zc && G <= hps::ZCOL32_MAX_G;
-      // the residual with z-column lanes as well (HPSINT_AMD_ZCOL_RES=0: not)
-      op->zcol_residual = op->zcol && env_int("HPSINT_AMD_ZCOL_RES", 1) != 0;
+      // the residual with z-column lanes as well (HPSINT_AMD_ZCOL_RES=0: not;
+      // with 5 and 6 order parameters only without a second history vector,
+      // see hps_residual)
+      op->zcol_residual = zc && G <= hps::ZCOL_RES_MAX_G && env_int("HPSINT_AMD_ZCOL_RES", 1) != 0;
       // FP64 tangent and residual: marches of up to HPSINT_AMD_ZCOL_MARCH
       // cache tiles (default 2: 32 layers, half the tile faces along z),
       // the deepest that still gives HPSINT_AMD_ZCOL_MARCH_WG (default 4)
@@ -374,6 +375,17 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
             op->zcol_mz = m * TZ;
             break;
           }
+      // FP64 tangent with 6 or 7 order parameters: only with two rounds of the
+      // marches that run at once; below that the emptier last round costs what
+      // the lanes save.  Corner lanes / z-column lanes, us, with 5, 6, 7 order
+      // parameters: 128^3 417 / 375, 456 / 422, 523 / 470; 160 x 150 x 170
+      // 808 / 737, 892 / 821, 1013 / 926; 90^3 (864 marches) 171 / 164,
+      // 184 / 187, 209 / 208; 61 x 75 x 67 (400) 71.9 / 71.7, 80 / 84,
+      // 95 / 95; 8 at 128^3 568 / 562 (spills), smaller meshes up to 18 %
+      // slower.
+      const int64_t marches = (int64_t)kp.nt[0] * op->ntz1 *
+                              ((ncm + op->zcol_mz - 1) / op->zcol_mz);
+      op->zcol = zc && (G <= 5 || (G <= hps::ZCOL_MAX_G && marches >= 4 * (int64_t)cus));
       if (op->zcol || op->zcol32)
         {
           for (const bool wide : {false, true})
@@ -660,7 +672,13 @@ extern "C" int hps_residual(hps_operator op, int wtd, double *dst, const double 
     HPS_HIP(hipEventRecord(timing_event(op, 0), op->stream));
   // with order 0 there is no history: evaluate without the history term
   const int w = (wtd == 2 && op->kp.order == 0) ? 1 : wtd;
-  const bool zres = op->zcol && !op->cut_active && op->zcol_residual;
+  // z-column lanes: with 5 and 6 order parameters the second history vector
+  // costs them more than the corner lanes.  Corner / z-column lanes, us, one
+  // history vector: 128^3 409 / 365 and 493 / 412, 90^3 159 / 149 and 194 /
+  // 172, 61 x 75 x 67 78.8 / 78.7 and 93 / 89 (7: 103 / 110); two: 128^3 448 /
+  // 455 and 532 / 500, 61 x 75 x 67 84 / 94 and 99 / 105.
+  const bool zres = op->zcol_residual && !op->cut_active &&
+                    (op->n_grains <= 4 || w < 2 || op->kp.order < 2);
   if (op->q2)
     op->q2->residual(q2_params(op), w, src, o[0], o[1], o[2], dst, op->stream);
   else if (zres)

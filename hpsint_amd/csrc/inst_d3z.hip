@@ -1,5 +1,5 @@
 // Instantiations: 3D Q1 scalar-mobility tangent with z-column lanes, FP64
-// with 1-4 order parameters, FP32 with 1-12; the residual with 1-4.
+// with 1-7 order parameters, FP32 with 1-12; the residual with 1-6.
 #include <cstdlib>
 
 #include "fe_q1_zcol.hpp"
@@ -64,6 +64,8 @@ namespace hps
         HPS_CASE(2)
         HPS_CASE(3)
         HPS_CASE(4)
+        HPS_CASE(5)
+        HPS_CASE(6)
 #undef HPS_CASE
         default:
           return false;

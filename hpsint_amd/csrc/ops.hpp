@@ -317,7 +317,9 @@ namespace hps
   // the 3D scalar-mobility tangent with z-column lanes (fe_q1_zcol.hpp):
   // 8 x 8 x tz tiles, ntz1 of them along y; reads the cache of the TX3 x
   // TY3 tiles.  False when n_grains is not built for it.
-  constexpr int ZCOL_MAX_G   = 4;  // FP64 tangent and the residual
+  // FP64 tangent: 216 registers with 5 order parameters, 256 with 7; 8 spill
+  constexpr int ZCOL_MAX_G     = 7;
+  constexpr int ZCOL_RES_MAX_G = 6; // the residual (FP64)
   constexpr int ZCOL32_MAX_G = 12; // FP32 tangent
   bool vmult_zcol_d3(int n_grains, const KParams &kp, int ntz1, int n_tiles, const double *src,
                      const double *cache, double *dst, double *part, hipStream_t s);

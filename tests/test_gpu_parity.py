@@ -544,3 +544,45 @@ def test_residual_zcol_and_corner_lanes(monkeypatch, zcol, cells, G):
         dst = op.initialize_dof_vector()
         op.evaluate_nonlinear_residual(dst, dev(u), wtd, old=[dev(o) for o in olds])
         assert rel_l2(host(dst), ref) <= TOL64, (wtd, rel_l2(host(dst), ref))
+
+
+@pytest.mark.parametrize("cells,G", [((19, 13, 37), 5), ((8, 9, 16), 5), ((9, 17, 5), 6),
+                                     ((1, 1, 1), 5), ((16, 8, 33), 6)])
+def test_zcol_five_and_six_order_parameters(cells, G):
+    """the tangent and, with at most one history vector, the residual at the
+    edges of the 8 x 8 tiles against the oracle, and the residual with two
+    (corner lanes), all at the tolerance of the FP64 comparisons"""
+    op, p = make_pair(3, cells, G, False, w0=100.0, w_hist=(-100.0,))
+    u = fields(p, 5)
+    src = np.random.default_rng(4).uniform(-1, 1, size=u.size)
+    ref = po.vmult(p, po.fill_qp(p, u), src)
+    op.fill_quadrature_point_values(dev(u))
+    dst = op.initialize_dof_vector()
+    op.vmult(dst, dev(src))
+    assert rel_l2(host(dst), ref) <= TOL64, rel_l2(host(dst), ref)
+    for hist in ((-100.0,), (-130.0, 30.0)):
+        op, p = make_pair(3, cells, G, False, w0=100.0, w_hist=hist)
+        olds = [fields(p, 6 + i) for i in range(len(hist))]
+        for wtd in (0, 1, 2):
+            ref = po.residual(p, wtd, u, olds)
+            dst = op.initialize_dof_vector()
+            op.evaluate_nonlinear_residual(dst, dev(u), wtd, old=[dev(o) for o in olds])
+            assert rel_l2(host(dst), ref) <= TOL64, (wtd, rel_l2(host(dst), ref))
+
+
+@pytest.mark.parametrize("cells,G", [((65, 128, 129), 6), ((128, 121, 64), 7), ((60, 64, 64), 7)])
+def test_zcol_six_and_seven_order_parameters_by_size(monkeypatch, cells, G):
+    """the tangent on meshes with and without enough marches for the z-column
+    lanes: the corner-lane kernel's result, which the small cases compare with
+    the oracle at the same tolerance"""
+    def tangent():
+        op, p = make_pair(3, cells, G, False, w0=100.0)
+        u = fields(p, 5)
+        op.fill_quadrature_point_values(dev(u))
+        dst = op.initialize_dof_vector()
+        op.vmult(dst, dev(np.random.default_rng(4).uniform(-1, 1, size=u.size)))
+        return host(dst)
+    got = tangent()
+    monkeypatch.setenv("HPSINT_AMD_ZCOL", "0")
+    ref = tangent()
+    assert rel_l2(got, ref) <= TOL64, rel_l2(got, ref)
