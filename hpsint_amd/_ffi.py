@@ -176,6 +176,7 @@ _SIGNATURES = {
     "hps_mlp_infer_workspace": [vp, ctypes.POINTER(i64)],
     "hps_mlp_infer": [vp, vp, vp, dbl, dbl, dbl, ctypes.POINTER(vp), ctypes.POINTER(vp), vp, vp,
                       vp, vp, vp],
+    "hps_mlp_infer_rows": [vp, dbl, dbl, dbl, vp, vp, vp],
     "hps_mlp_predict": [vp, vp, vp, vp, vp, vp, vp, vp],
     "hps_mlp_targets": [vp, vp, vp, vp, vp, vp, vp, vp],
 }

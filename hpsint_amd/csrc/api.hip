@@ -1632,6 +1632,24 @@ extern "C" int hps_mlp_infer(hps_operator op, const double *u_prev, const double
   return HPS_OK;
 }
 
+extern "C" int hps_mlp_infer_rows(hps_operator op, double dt, double dt_scale, double inc_scale,
+                                  const int *top2, const void *workspace, void *X)
+{
+  if (int r = check_op(op))
+    return r;
+  if (!top2 || !workspace || !X)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "mlp_infer_rows: null argument");
+  const hps::FeatParams fp = feat_params(op, dt, dt_scale, inc_scale);
+  if (hps::mlp_infer_workspace(fp) == 0)
+    return fail(HPS_ERR_UNSUPPORTED, "mlp_infer_rows: mesh too large");
+  if (((uintptr_t)workspace | (uintptr_t)X) & 15)
+    return fail(HPS_ERR_INVALID_ARGUMENT,
+                "mlp_infer_rows: workspace and X must be 16-byte aligned");
+  hps::mlp_infer_rows(op->stream, fp, top2, workspace, (uint16_t *)X);
+  HPS_LAUNCHED();
+  return HPS_OK;
+}
+
 extern "C" int hps_mlp_predict(hps_operator op, const double *u_prev, const double *u_cur,
                                const float *Y, const int *top2, const float *out_scale,
                                const float *lscale, double *u_pred)

@@ -14,7 +14,8 @@
 //   k_loss      MSE and its gradient
 //   k_adam      Adam step on FP32 master weights + BF16 copies
 //   k_predict   applies the corrections to the extrapolated state
-// The stencil features and the fused inference are in mlp_infer.hip.
+// The stencil features are in mlp_features.hip, the fused inference in
+// mlp_infer.hip, the fused training step in mlp_train.hip.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

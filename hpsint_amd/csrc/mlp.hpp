@@ -44,6 +44,9 @@ namespace hps
   void    mlp_infer(hipStream_t, const FeatParams &, const double *u_prev, const double *u_cur,
                     const uint16_t *const *W, const float *const *b, const float *out_scale,
                     int *top2, float *lscale, double *out, void *ws);
+  // the feature rows (as mlp_features) that the last mlp_infer on ws formed
+  void    mlp_infer_rows(hipStream_t, const FeatParams &, const int *top2, const void *ws,
+                         uint16_t *X);
   // one Adam step of the 272-128-128-128-4 network on M rows; returns the
   // device address of the loss' partial sums (n_loss of them).  X, Wb and ws
   // 16-byte aligned

@@ -428,6 +428,74 @@ namespace hps
       }
   }
 
+  // feature rows (mlp_features.hip) of the nodes of the last k_fields, from its
+  // arrays instead of u: for programs that look at the rows of a prediction.  32
+  // nodes per workgroup, 8 lanes per node; the sums of squares in k_features'
+  // order, so that both give the same bits.
+  constexpr int ROW_NODES = 32;
+  __global__ void __launch_bounds__(256) k_rows(InferArgs a, uint16_t *__restrict__ X)
+  {
+    constexpr int XS = NET_IN + 8;
+    __shared__ __align__(16) uint16_t rows[ROW_NODES * XS];
+    const int64_t N = a.fp.n_nodes, n0 = (int64_t)blockIdx.x * ROW_NODES;
+    const int     r = threadIdx.x >> 3, sub = threadIdx.x & 7;
+    const int64_t node = min(n0 + r, N - 1);
+    const int     nx = a.fp.nn[0], ny = a.fp.nn[1], nz = a.fp.nn[2];
+    const int     x = (int)(node % nx), y = (int)(node / nx % ny), z = (int)(node / nx / ny);
+    const double   *d2 = (const double *)(a.ws + a.l.d2), *ds = (const double *)(a.ws + a.l.ds);
+    const uint16_t *v4 = (const uint16_t *)(a.ws + a.l.v4), *be = (const uint16_t *)(a.ws + a.l.be);
+    const double   *de = (const double *)(a.ws + a.l.de);
+    auto            plane = [&](int i) { return min(max(i, 0), a.fp.n_comp - 3) * N; };
+    const int64_t   p1 = plane(a.top2[2 * node]), p2 = plane(a.top2[2 * node + 1]);
+    auto            at = [&](int s) {
+      const int xx = min(max(x + s % 3 - 1, 0), nx - 1), yy = min(max(y + s / 3 % 3 - 1, 0), ny - 1);
+      const int zz = min(max(z + s / 9 - 1, 0), nz - 1);
+      return ((int64_t)zz * ny + yy) * nx + xx;
+    };
+    double ss = 0.0;
+    for (int s = sub; s < 27; s += 8)
+      {
+        const int64_t q    = at(s);
+        const double  d[5] = {d2[2 * q], d2[2 * q + 1], ds[q], de[p1 + q], de[p2 + q]};
+#pragma unroll
+        for (int f = 0; f < 5; ++f)
+          ss += d[f] * d[f];
+      }
+    ss += __shfl_xor(ss, 1, 64);
+    ss += __shfl_xor(ss, 2, 64);
+    ss += __shfl_xor(ss, 4, 64);
+    const double ls = sqrt(ss / 135.0) + a.fp.inc_floor, inv = 1.0 / ls;
+    uint16_t    *row = rows + r * XS;
+    for (int s = sub; s < 27; s += 8)
+      {
+        const int64_t q  = at(s);
+        uint16_t     *o  = row + 10 * s;
+        o[0] = v4[4 * q];
+        o[1] = v4[4 * q + 1];
+        o[2] = v4[4 * q + 2];
+        o[3] = be[p1 + q];
+        o[4] = be[p2 + q];
+        o[5] = f2bf((float)(d2[2 * q] * inv));
+        o[6] = f2bf((float)(d2[2 * q + 1] * inv));
+        o[7] = f2bf((float)(ds[q] * inv));
+        o[8] = f2bf((float)(de[p1 + q] * inv));
+        o[9] = f2bf((float)(de[p2 + q] * inv));
+      }
+    if (sub == 0)
+      {
+        row[270] = f2bf((float)(a.fp.dt * a.fp.dt_scale));
+        row[271] = f2bf((float)log10(ls * a.fp.inc_scale));
+      }
+    __syncthreads();
+    constexpr int CH = NET_IN / 8; // 16-byte pieces of a row
+    for (int i = threadIdx.x; i < ROW_NODES * CH; i += 256)
+      {
+        const int m = i / CH, c = i - CH * m;
+        if (n0 + m < N)
+          *(uint4 *)(X + (n0 + m) * NET_IN + 8 * c) = *(const uint4 *)(rows + m * XS + 8 * c);
+      }
+  }
+
   int64_t mlp_infer_workspace(const FeatParams &fp)
   {
     // k_infer's 32-bit byte offsets must reach every array of the workspace
@@ -471,5 +539,16 @@ namespace hps
         HPS_NC(9) HPS_NC(10) HPS_NC(11) HPS_NC(12) HPS_NC(13) HPS_NC(14)
 #undef HPS_NC
       }
+  }
+
+  void mlp_infer_rows(hipStream_t s, const FeatParams &fp, const int *top2, const void *ws,
+                      uint16_t *X)
+  {
+    InferArgs a{};
+    a.fp   = fp;
+    a.top2 = const_cast<int *>(top2);
+    a.ws   = (char *)const_cast<void *>(ws);
+    a.l    = infer_ws(fp.n_nodes, fp.n_comp - 2);
+    k_rows<<<(unsigned)((fp.n_nodes + ROW_NODES - 1) / ROW_NODES), 256, 0, s>>>(a, X);
   }
 } // namespace hps

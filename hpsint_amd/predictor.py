@@ -170,6 +170,7 @@ class LearnedPredictor:
         n = op.n_nodes
         self._X = None
         self._ws = None
+        self._inferred = None   # dt and scales of the last fused prediction
         self.top2 = torch.empty(n, 2, dtype=torch.int32, device=dev)
         self.lscale = torch.empty(n, dtype=torch.float32, device=dev)
         self.use_network = True
@@ -177,12 +178,23 @@ class LearnedPredictor:
 
     @property
     def X(self):
-        """feature rows of the last features() call (allocated by the first
-        use: the fused inference keeps no rows)"""
+        """feature rows of the last features() or predict() call.  The fused
+        inference forms them in registers: they are written when they are first
+        asked for, and from then on by each prediction"""
         if self._X is None:
             self._X = torch.empty(self.op.n_nodes, N_IN, dtype=torch.bfloat16,
                                   device=self.mlp.W[0].device)
+            if self._inferred is not None:
+                self._write_rows()
         return self._X
+
+    @X.setter
+    def X(self, rows):
+        self._X = rows
+
+    def _write_rows(self):
+        check(lib().hps_mlp_infer_rows(self.op.handle, *self._inferred, _p(self.top2),
+                                       _p(self._ws), _p(self._X)))
 
     def step_scale(self, u_prev, u_cur):
         """RMS of u_cur - u_prev, computed by the library"""
@@ -193,6 +205,7 @@ class LearnedPredictor:
 
     def features(self, u_prev, u_cur, dt):
         self.inc_scale = 1.0 / self.step_scale(u_prev, u_cur)
+        self._inferred = None
         check(lib().hps_mlp_features(self.op.handle, _p(u_prev), _p(u_cur), dt, self.dt_scale,
                                      self.inc_scale, _p(self.X), _p(self.top2),
                                      _p(self.lscale)))
@@ -224,6 +237,9 @@ class LearnedPredictor:
                 arr(*[w.data_ptr() for w in self.mlp.Wb]),
                 arr(*[b.data_ptr() for b in self.mlp.b]), _p(self.out_scale), _p(self.top2),
                 _p(self.lscale), _p(out), _p(ws)))
+            self._inferred = (dt, self.dt_scale, self.inc_scale)
+            if self._X is not None:
+                self._write_rows()
             return out
         if self.use_network:
             X, _ = self.features(u_prev, u_cur, dt)

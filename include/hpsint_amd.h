@@ -386,6 +386,12 @@ int hps_mlp_infer(hps_operator op, const double *u_prev, const double *u_cur, do
                   double dt_scale, double inc_scale, const void *const *W,
                   const float *const *b, const float *out_scale, int *top2, float *lscale,
                   double *u_pred, void *workspace);
+/* The feature rows (X: n_nodes x 272 bf16, 16-byte aligned, as
+ * hps_mlp_features) that the last hps_mlp_infer on this workspace formed in
+ * registers, from that call's workspace, top2, dt and scales: u_prev and u_cur
+ * may have changed since. */
+int hps_mlp_infer_rows(hps_operator op, double dt, double dt_scale, double inc_scale,
+                       const int *top2, const void *workspace, void *X);
 /* training targets: (u_next - (2 u_cur - u_prev)) / (ls * out_scale) on the
  * 4 outputs */
 int hps_mlp_targets(hps_operator op, const double *u_prev, const double *u_cur,

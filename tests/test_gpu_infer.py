@@ -94,6 +94,33 @@ def test_fused_inference_not_in_place():
             p(cur.data_ptr()), p(pred._ws.data_ptr())))
 
 
+# 32 nodes per workgroup: fewer, a remainder, a mesh of one node plane
+@pytest.mark.parametrize("cells,G", [((1, 1, 1), 1), ((7, 5, 9), 4), ((9, 10, 4), 12),
+                                     ((31, 6), 3)])
+def test_rows_of_a_prediction(cells, G):
+    """X after predict holds that prediction's feature rows, bit for bit those
+    of features(): asked for afterwards, with the inputs overwritten in
+    between, and as a tensor that the program already holds"""
+    op, pred, prev, cur = setup(cells, G)
+    other = LearnedPredictor(op, pred.mlp, dt_scale=1e3)
+    out = torch.empty_like(cur)
+    want, _ = other.features(prev, cur, 1e-3)
+    want = want.clone()
+    pred.predict(prev, cur, 1e-3, out)
+    prev2, cur2 = prev * 0.9, cur * 1.01
+    prev.fill_(7.0)
+    cur.fill_(5.0)
+    rows = pred.X
+    assert torch.isfinite(rows).all() and torch.equal(rows, want)
+    want2, _ = other.features(prev2, cur2, 2e-3)
+    pred.predict(prev2, cur2, 2e-3, out)
+    assert pred.X is rows and torch.equal(rows, want2)
+    mine = torch.zeros_like(rows)
+    pred.X = mine
+    pred.predict(prev2, cur2, 2e-3, out)
+    assert torch.equal(mine, want2)
+
+
 @pytest.mark.parametrize("n", [1, 255, 256, 524289])
 def test_norm2_diff(n):
     op, _, _, _ = setup((3, 3, 3), 1)
