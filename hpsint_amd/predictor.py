@@ -22,6 +22,17 @@ N_IN = 272
 N_OUT = 4
 
 
+# the methods that the fused calls stand for
+_OWN = {}
+
+
+def _unchanged(obj, cls):
+    """obj is a cls whose methods behind the fused calls are the class's own: a
+    subclass or a program that replaces one of them gets it called"""
+    return isinstance(obj, cls) and all(
+        getattr(getattr(obj, name), "__func__", None) is f for name, f in _OWN[cls].items())
+
+
 def _p(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
@@ -124,8 +135,9 @@ class MLP:
 
     def _train_fused(self, X, T, M, lr, b1=0.9, b2=0.999, eps=1e-8):
         """hps_mlp_train_step, or None where it does not cover the call:
-        other widths, more rows than it takes or unaligned operands"""
-        if self.dims != [N_IN, 128, 128, 128, N_OUT]:
+        other widths, more rows than it takes, unaligned operands or a method
+        of its own for a part of the step"""
+        if not _unchanged(self, MLP) or self.dims != [N_IN, 128, 128, 128, N_OUT]:
             return None
         n = ctypes.c_int64()
         check(lib().hps_mlp_train_workspace(self.op.handle, M, ctypes.byref(n)))
@@ -213,11 +225,13 @@ class LearnedPredictor:
 
     def _infer_workspace(self, u_prev, u_cur, out):
         """the workspace of hps_mlp_infer, or None where that call does not
-        cover the prediction: other widths than the built network's, an
-        output that overlaps an input (its stencils read the inputs while
-        others' results are written) or a mesh beyond its 32-bit offsets"""
+        cover the prediction: other widths than the built network's, a
+        network or features() of the program's own, an output that overlaps an
+        input (its stencils read the inputs while others' results are written)
+        or a mesh beyond its 32-bit offsets"""
         size = 8 * self.op.n_dofs
-        if (self.mlp.dims != [N_IN, 128, 128, 128, N_OUT]
+        if (not _unchanged(self, LearnedPredictor) or not _unchanged(self.mlp, MLP)
+                or self.mlp.dims != [N_IN, 128, 128, 128, N_OUT]
                 or any(abs(out.data_ptr() - u.data_ptr()) < size for u in (u_prev, u_cur))):
             return None
         if self._ws is None:
@@ -261,3 +275,9 @@ class LearnedPredictor:
         if len(states) < 2:
             return x
         return self.predict(states[1], states[0], dt, x)
+
+
+_OWN.update({
+    MLP: {n: getattr(MLP, n) for n in ("forward", "loss_grad", "backward", "adam")},
+    LearnedPredictor: {"features": LearnedPredictor.features},
+})
