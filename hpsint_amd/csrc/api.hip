@@ -1101,31 +1101,45 @@ extern "C" int hps_precond_get_blocks(hps_operator op, double *blocks)
 }
 
 // ------------------------------------------------------------------ BLAS-1
+// whether a waiting host thread may hold its core: not where the process chose
+// blocking or yielding waits for the device (hipSetDeviceFlags)
+static bool may_spin()
+{
+  unsigned flags = 0;
+  if (hipGetDeviceFlags(&flags) != hipSuccess)
+    {
+      (void)hipGetLastError();
+      return true;
+    }
+  return !(flags & (hipDeviceScheduleBlockingSync | hipDeviceScheduleYield));
+}
+
+static void spin_pause()
+{
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+  __builtin_ia32_pause();
+#endif
+}
+
 // waits until the device has raised the flag to red_seq.  The host polls the
-// pinned flag (a stream synchronisation takes about 10 us more); now and then
-// it asks for the stream's state, so that a failed launch ends the wait.
+// pinned flag (a stream synchronisation takes about 10 us more) for about a
+// millisecond, which covers an iteration's reductions; behind longer work, or
+// where the process chose waits that leave the core, it synchronises the
+// stream, which also reports a launch that failed.
 static int wait_flag(hps_operator op)
 {
-  const unsigned seq = op->red_seq;
-  for (unsigned spin = 1;; ++spin)
-    {
-      if (__atomic_load_n(op->red_flag, __ATOMIC_ACQUIRE) == seq)
-        return HPS_OK;
-      if (spin % 4096 != 0)
-        continue;
-      const hipError_t e = hipStreamQuery(op->stream);
-      if (e == hipErrorNotReady)
-        {
-          (void)hipGetLastError();
-          continue;
-        }
-      if (e != hipSuccess)
-        return fail(HPS_ERR_HIP, std::string("reduction: ") + hipGetErrorString(e));
-      // all work is done: the flag is up, or the kernel did not run
-      if (__atomic_load_n(op->red_flag, __ATOMIC_ACQUIRE) == seq)
-        return HPS_OK;
-      return fail(HPS_ERR_HIP, "reduction: the result was not delivered");
-    }
+  constexpr int  POLLS = 20000; // about 50 ns each
+  const unsigned seq   = op->red_seq;
+  auto           up    = [&] { return __atomic_load_n(op->red_flag, __ATOMIC_ACQUIRE) == seq; };
+  if (may_spin())
+    for (int i = 0; i < POLLS; ++i)
+      {
+        if (up())
+          return HPS_OK;
+        spin_pause();
+      }
+  HPS_HIP(hipStreamSynchronize(op->stream));
+  return up() ? HPS_OK : fail(HPS_ERR_HIP, "reduction: the result was not delivered");
 }
 
 // k <= 64 results of red_out on the host

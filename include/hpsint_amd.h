@@ -13,8 +13,11 @@
  *
  * Every call is enqueued on the operator's stream (hps_set_stream) and
  * returns without waiting, except the reductions that return a value to the
- * host (hps_dot, hps_norm2, hps_multi_dot, hps_sync).  Calls on one handle
- * must not overlap from several host threads.
+ * host (hps_dot, hps_norm2, hps_multi_dot, ...) and hps_sync.  The reductions
+ * poll a flag that the device raises, which keeps the host thread's core busy
+ * for up to about a millisecond, and then synchronise the stream; where the
+ * process chose blocking or yielding waits (hipSetDeviceFlags) they do so at
+ * once.  Calls on one handle must not overlap from several host threads.
  *
  * Return value: HPS_OK or one of the error codes below; hps_last_error()
  * gives the message of the last failure on the calling thread.
