@@ -144,6 +144,8 @@ _SIGNATURES = {
     "hps_multi_axpy_norm": [vp, i64, cint, vp, pd, vp, pd],
     "hps_convert_f64_to_f32": [vp, i64, vp, vp],
     "hps_norm2_f32": [vp, i64, vp, pd],
+    "hps_orthogonalise": [vp, i64, cint, vp, vp, pd, pd],
+    "hps_orthogonalise_f32": [vp, i64, cint, vp, vp, pd, pd],
     "hps_multi_dot_f32": [vp, i64, cint, vp, vp, pd],
     "hps_multi_axpy_norm_f32": [vp, i64, cint, vp, pd, vp, pd],
     "hps_scale_f32": [vp, i64, dbl, vp],

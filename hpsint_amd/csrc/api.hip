@@ -1155,33 +1155,6 @@ static int fetch(hps_operator op, int k, double *result)
   return HPS_OK;
 }
 
-// Gram-Schmidt step of GMRES (solver.hip): h[j] = <V_j, w>, w -= sum h_j V_j,
-// *norm = |w|, w /= |w| (unless 0), with one wait
-template <typename T>
-static int gram_schmidt(hps_operator op, int64_t n, int k, const T *V, T *w, double *h,
-                        double *norm)
-{
-  hps::blas_gram_schmidt<T>(op->stream, n, k, V, w, op->red_partial, op->red_out, op->red_host,
-                            op->red_host + hps::MAXK, op->red_flag, ++op->red_seq);
-  HPS_LAUNCHED();
-  if (int r = wait_flag(op))
-    return r;
-  for (int j = 0; j < k; ++j)
-    h[j] = op->red_host[j];
-  *norm = op->red_host[hps::MAXK];
-  return HPS_OK;
-}
-int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const double *V, double *w,
-                              double *h, double *norm)
-{
-  return gram_schmidt<double>(op, n, k, V, w, h, norm);
-}
-int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const float *V, float *w,
-                              double *h, double *norm)
-{
-  return gram_schmidt<float>(op, n, k, V, w, h, norm);
-}
-
 extern "C" int hps_dot(hps_operator op, int64_t n, const double *x, const double *y,
                        double *result)
 {
@@ -1242,6 +1215,48 @@ extern "C" int hps_multi_axpy_norm(hps_operator op, int64_t n, int k, const doub
   hps::blas_multi_axpy_norm(op->stream, n, k, V, op->red_out + 32, w, op->red_partial,
                             op->red_out);
   return fetch(op, 1, norm);
+}
+
+// Classical Gram-Schmidt with one wait per pass; the second pass, when one is
+// due, starts from the unscaled rest and adds to h
+template <typename T>
+static int orthogonalise(hps_operator op, int64_t n, int k, const T *V, T *w, double *h,
+                         double *norm)
+{
+  if (int r = check_op(op))
+    return r;
+  if (k < 1 || k > hps::MAXK)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "orthogonalise: k must be 1..32");
+  if (!V || !w || !h || !norm)
+    return fail(HPS_ERR_INVALID_ARGUMENT, "orthogonalise: null argument");
+  const double *res = op->red_host + hps::MAXK;
+  for (int pass = 0; pass < 2; ++pass)
+    {
+      hps::blas_gram_schmidt<T>(op->stream, n, k, V, w, op->red_partial, op->red_out, pass == 1,
+                                op->red_host, op->red_host + hps::MAXK, op->red_flag,
+                                ++op->red_seq);
+      HPS_LAUNCHED();
+      if (int r = wait_flag(op))
+        return r;
+      for (int j = 0; j < k; ++j)
+        h[j] = pass ? h[j] + op->red_host[j] : op->red_host[j];
+      *norm = res[0];
+      if (res[1] == 0.0)
+        break;
+    }
+  return HPS_OK;
+}
+
+extern "C" int hps_orthogonalise(hps_operator op, int64_t n, int k, const double *V, double *w,
+                                 double *h, double *norm)
+{
+  return orthogonalise<double>(op, n, k, V, w, h, norm);
+}
+
+extern "C" int hps_orthogonalise_f32(hps_operator op, int64_t n, int k, const float *V, float *w,
+                                     double *h, double *norm)
+{
+  return orthogonalise<float>(op, n, k, V, w, h, norm);
 }
 
 extern "C" int hps_axpy(hps_operator op, int64_t n, double a, const double *x, double *y)

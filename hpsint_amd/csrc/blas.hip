@@ -293,14 +293,20 @@ namespace hps
   }
 
   // w /= norm (as w times 1 / norm; left alone if 0), the norm read from
-  // memory or (ROWS) from nb partial sums of squares.  The first block also
-  // sends h and the norm to the host and raises the flag.
+  // memory or (ROWS) from nb partial sums of squares.  Unless this is the last
+  // pass, a w that lost more than half of its norm sqrt(|w|^2 + |h|^2) (V
+  // orthonormal) is left as it is: it goes through another pass and is rounded
+  // to T once for the normalisation, not twice (and not read and written for
+  // nothing: 22.5 us at 129^3 nodes, 6 components, FP32).  The first block also
+  // sends h, the norm and whether another pass is due (1 or 0) to the host and
+  // raises the flag.
   template <typename T, bool ROWS>
   __global__ void __launch_bounds__(RB)
     k_scale_norm(int64_t n, T *__restrict__ w, const double *__restrict__ norm, int nb, int k,
-                 const double *__restrict__ h, double *host_h, double *host_norm, unsigned *flag,
-                 unsigned seq)
+                 const double *__restrict__ h, int last, double *host_h, double *host_norm,
+                 unsigned *flag, unsigned seq)
   {
+    static_assert(MAXK <= 64, "a coefficient per lane");
     __shared__ double sh[1];
     double            v;
     if constexpr (ROWS)
@@ -310,18 +316,28 @@ namespace hps
       }
     else
       v = norm[0];
+    const int    lane = threadIdx.x & 63;
+    const double hj   = lane < k ? h[lane] : 0.0;
+    double       hh   = hj * hj;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+      hh += __shfl_xor(hh, o, 64);
+    const bool again = !last && v > 0.0 && v < 0.5 * sqrt(v * v + hh);
     if (blockIdx.x == 0)
       {
         if ((int)threadIdx.x < k)
-          host_h[threadIdx.x] = h[threadIdx.x];
+          host_h[threadIdx.x] = hj;
         if (threadIdx.x == 0)
-          *host_norm = v;
+          {
+            host_norm[0] = v;
+            host_norm[1] = again ? 1.0 : 0.0;
+          }
         __syncthreads();
         __threadfence_system();
         if (threadIdx.x == 0)
           raise_flag(flag, seq);
       }
-    if (v == 0.0)
+    if (again || v == 0.0)
       return;
     const double a = 1.0 / v;
     for (int64_t i = (int64_t)blockIdx.x * RB + threadIdx.x; i < n; i += (int64_t)gridDim.x * RB)
@@ -832,8 +848,8 @@ namespace hps
 
   template <typename T>
   void blas_gram_schmidt(hipStream_t s, int64_t n, int k, const T *V, T *w, double *partial,
-                         double *out, double *host_h, double *host_norm, unsigned *flag,
-                         unsigned seq)
+                         double *out, bool last, double *host_h, double *host_norm,
+                         unsigned *flag, unsigned seq)
   {
     const int  nb  = red_blocks(n);
     const bool inl = nb <= GS_INLINE_BLOCKS;
@@ -859,16 +875,17 @@ namespace hps
       }
     const int g = inl ? nb : grid_for(n, 256 * 4);
     if (inl)
-      k_scale_norm<T, true><<<g, RB, 0, s>>>(n, w, pn, nb, k, out, host_h, host_norm, flag, seq);
+      k_scale_norm<T, true>
+        <<<g, RB, 0, s>>>(n, w, pn, nb, k, out, last, host_h, host_norm, flag, seq);
     else
       k_scale_norm<T, false>
-        <<<g, RB, 0, s>>>(n, w, out + MAXK, nb, k, out, host_h, host_norm, flag, seq);
+        <<<g, RB, 0, s>>>(n, w, out + MAXK, nb, k, out, last, host_h, host_norm, flag, seq);
   }
   template void blas_gram_schmidt<double>(hipStream_t, int64_t, int, const double *, double *,
-                                          double *, double *, double *, double *, unsigned *,
+                                          double *, double *, bool, double *, double *, unsigned *,
                                           unsigned);
   template void blas_gram_schmidt<float>(hipStream_t, int64_t, int, const float *, float *,
-                                         double *, double *, double *, double *, unsigned *,
+                                         double *, double *, bool, double *, double *, unsigned *,
                                          unsigned);
 
   void blas_multi_dot(hipStream_t s, int64_t n, int k, const double *V, const double *w,

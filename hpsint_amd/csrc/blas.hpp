@@ -31,14 +31,15 @@ namespace hps
                       double *partial, double *out);
   void blas_multi_axpy_norm(hipStream_t, int64_t n, int k, const double *V, const double *h,
                             double *w, double *partial, double *out);
-  // One classical Gram-Schmidt step: h[j] = <V_j, w>, w -= sum h_j V_j,
-  // norm = |w|, w /= norm (left alone if 0).  h (k values), norm and then
-  // *flag = seq are written to pinned host memory; scratch: partial (RED_BLOCKS x
-  // k values) and out (MAXK + 8)
+  // One pass of classical Gram-Schmidt: h[j] = <V_j, w>, w -= sum h_j V_j,
+  // norm = |w|, and w /= norm unless norm is 0 or (last false) another pass is
+  // due.  h (k values) and host_norm (the norm, then 1 if another pass is due,
+  // else 0) and then *flag = seq are written to pinned host memory; scratch:
+  // partial (RED_BLOCKS x k values) and out (MAXK + 8)
   template <typename T>
   void blas_gram_schmidt(hipStream_t, int64_t n, int k, const T *V, T *w, double *partial,
-                         double *out, double *host_h, double *host_norm, unsigned *flag,
-                         unsigned seq);
+                         double *out, bool last, double *host_h, double *host_norm,
+                         unsigned *flag, unsigned seq);
   // k <= 64 results from device memory to pinned host memory, then *flag = seq
   void publish(hipStream_t, int k, const double *out, double *host, unsigned *flag, unsigned seq);
   void blas_axpy(hipStream_t, int64_t n, double a, const double *x, double *y);

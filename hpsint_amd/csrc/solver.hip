@@ -36,12 +36,6 @@ struct hps_newton_s
 
 // error reporting shared with the operator entry points (api.hip)
 int hps_internal_fail(int code, const char *msg);
-// one Gram-Schmidt step with one wait (api.hip): h[j] = <V_j, w>, w -= sum h_j
-// V_j, *norm = |w|, w /= |w| (unless 0)
-int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const double *V, double *w,
-                              double *h, double *norm);
-int hps_internal_gram_schmidt(hps_operator op, int64_t n, int k, const float *V, float *w,
-                              double *h, double *norm);
 
 namespace
 {
@@ -132,31 +126,6 @@ namespace
     }
   };
 
-  // Classical Gram-Schmidt against k vectors with one re-orthogonalisation
-  // pass when the new vector loses more than half of its norm: h, the norm,
-  // and w normalised (unless its norm is 0).  The second pass starts from the
-  // normalised vector, so its coefficients and norm scale by the first norm.
-  template <typename T>
-  int orthogonalise(hps_operator op, int64_t n, int k, const T *V, T *w, double *h,
-                    double *norm)
-  {
-    HPS_TRY(hps_internal_gram_schmidt(op, n, k, V, w, h, norm));
-    // norm before the projection, sqrt(|w'|^2 + |h|^2) (V orthonormal)
-    double hh = 0.0;
-    for (int i = 0; i < k; ++i)
-      hh += h[i] * h[i];
-    if (*norm > 0.0 && *norm < 0.5 * std::sqrt(*norm * *norm + hh))
-      {
-        std::vector<double> h2(k);
-        double              n2 = 0.0;
-        HPS_TRY(hps_internal_gram_schmidt(op, n, k, V, w, h2.data(), &n2));
-        for (int i = 0; i < k; ++i)
-          h[i] += *norm * h2[i];
-        *norm *= n2;
-      }
-    return HPS_OK;
-  }
-
   // Restarted GMRES(m) with left preconditioning and classical Gram-Schmidt
   // (one re-orthogonalisation pass when the new vector loses more than
   // half of its norm); convergence as deal.II's ReductionControl on the
@@ -205,7 +174,7 @@ namespace
             double *vj1 = V + (int64_t)(j + 1) * n;
             HPS_TRY(apply_prec_op(nt, V + (int64_t)j * n, vj1));
             double wnorm = 0.0;
-            HPS_TRY(orthogonalise(op, n, j + 1, V, vj1, a.h.data(), &wnorm));
+            HPS_TRY(hps_orthogonalise(op, n, j + 1, V, vj1, a.h.data(), &wnorm));
             a.h[j + 1]       = wnorm;
             const double res = a.add_column(j);
             ++it;
@@ -286,7 +255,7 @@ namespace
             HPS_TRY(hps_vmult_f32(op, nt->y32, V + (int64_t)j * n));
             HPS_TRY(hps_precond_apply_f32(op, vj1, nt->y32));
             double wnorm = 0.0;
-            HPS_TRY(orthogonalise(op, n, j + 1, V, vj1, a.h.data(), &wnorm));
+            HPS_TRY(hps_orthogonalise_f32(op, n, j + 1, V, vj1, a.h.data(), &wnorm));
             a.h[j + 1]       = wnorm;
             const double res = a.add_column(j);
             ++it;

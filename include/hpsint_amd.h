@@ -219,6 +219,12 @@ int hps_multi_dot_noalloc(void *stream, int64_t n, int k, const double *V, const
 /* w -= sum_j h[j] V_j, then returns ||w|| (fused CGS update + norm) */
 int hps_multi_axpy_norm(hps_operator op, int64_t n, int k, const double *V,
                         const double *h, double *w, double *norm);
+/* w made orthogonal to the k (1..32) vectors of V (orthonormal, back to back)
+ * by classical Gram-Schmidt and normalised: on return the old w is sum_j h[j]
+ * V_j + norm w, |w| = 1 (w = 0 if norm is 0).  A second pass runs when the first
+ * leaves less than half of w's norm. */
+int hps_orthogonalise(hps_operator op, int64_t n, int k, const double *V, double *w, double *h,
+                      double *norm);
 /* y += sum_{j<k} a[j] V_j (the GMRES solution update x += V y; a on the
  * host, V as in hps_multi_dot) */
 int hps_axpy_multi(hps_operator op, int64_t n, int k, const double *a, const double *V,
@@ -237,6 +243,8 @@ int hps_multi_dot_f32(hps_operator op, int64_t n, int k, const float *V, const f
                       double *h);
 int hps_multi_axpy_norm_f32(hps_operator op, int64_t n, int k, const float *V,
                             const double *h, float *w, double *norm);
+int hps_orthogonalise_f32(hps_operator op, int64_t n, int k, const float *V, float *w,
+                          double *h, double *norm);
 int hps_scale_f32(hps_operator op, int64_t n, double a, float *x);
 /* y (FP64) += sum_{j<k} a[j] X_j (FP32 vectors X + j*n), FP64 arithmetic */
 int hps_axpy_multi_f32(hps_operator op, int64_t n, int k, const double *a, const float *X,
