@@ -239,7 +239,12 @@ namespace hps
   //   grad row of c = M grad(dmu) + s grad(mu_lin),
   //   s = dM/dc dc + 2 Mgb sum_i (sum_j eta_j - eta_i) deta_i,
   //   dM/dc = 30 (Mvol - Mvap) p^2 + 8 Msurf p (1 - 2 c), p = c (1 - c).
-  // The sums over pairs and over j != i are formed from running sums, O(G).
+  // Both sums are formed from running sums, O(G), the second as the sum over
+  // pairs of eta_i deta_j + eta_j deta_i: as (sum eta)(sum deta) - sum eta deta,
+  // an operation per i less, it cancels where one grain dominates (eta = 1 and 0,
+  // deta = 1 and 1e-5: an FP32 error of 1e-3 of the result).  A second loop with
+  // sum_j eta_j - eta_i needs no more operations than that, but holds eta and
+  // deta for longer: 1766 us at 160^3, 12 order parameters, FP64, against 1638.
   template <int G, typename T, typename PP>
   __device__ __forceinline__ void scalar_mobility_terms(const PP &pp, T c,
                                                         const T *etas, const T *v, T &M,
@@ -247,19 +252,20 @@ namespace hps
   {
     // (no order parameter is active in some tiles of the cut-off: G = 0)
     T sum = G > 0 ? etas[0] : T(0.0), sv = G > 0 ? v[2] : T(0.0);
-    T ev = sum * sv, pairs = T(0.0);
+    T pairs = T(0.0), factor = T(0.0);
 #pragma unroll
     for (int i = 1; i < G; ++i)
       {
         pairs += etas[i] * sum;
+        factor += etas[i] * sv;
+        factor += v[2 + i] * sum;
         sum += etas[i];
-        ev += etas[i] * v[2 + i];
         sv += v[2 + i];
       }
     const T p    = c * (T(1.0) - c);
     M            = scalar_mobility(pp, c, p, pairs);
     const T dMdc = p * (pp_dM30<T>(pp) * p + pp_Ms8<T>(pp) * (T(1.0) - T(2.0) * c));
-    s            = dMdc * v[0] + pp_Mgb2<T>(pp) * (sum * sv - ev);
+    s            = dMdc * v[0] + pp_Mgb2<T>(pp) * factor;
   }
 
   // qsum (optional, tensorial only): sum_i deta_i Q_i formed by the caller,

@@ -586,3 +586,39 @@ def test_zcol_six_and_seven_order_parameters_by_size(monkeypatch, cells, G):
     monkeypatch.setenv("HPSINT_AMD_ZCOL", "0")
     ref = tangent()
     assert rel_l2(got, ref) <= TOL64, rel_l2(got, ref)
+
+
+@pytest.mark.parametrize("zcol", ["0", "1"])
+@pytest.mark.parametrize("cells,G", [((9, 8, 10), 2), ((9, 8, 10), 4), ((9, 8, 10), 5),
+                                     ((9, 8, 10), 8), ((9, 8, 10), 12), ((20, 17), 2),
+                                     ((20, 17), 6)])
+def test_mobility_derivative_in_a_grain(monkeypatch, cells, G, zcol):
+    """the c row in a single grain (c = eta_1 = 1) with grad mu = 1 along x, for
+    deta_1 = 1 and deta_2 = 1e-5: its coefficient 2 Mgb sum_i (sum_j eta_j -
+    eta_i) deta_i is 2e-5 Mgb, without a trace of the large deta_1.  The row is
+    that coefficient times +-(the face's weight) on the two faces x = const and
+    0 elsewhere.  Interpolation, gradient, coefficient and sums over 8 cells
+    round some 60 times: 64 halves of the type's spacing."""
+    monkeypatch.setenv("HPSINT_AMD_ZCOL", zcol)
+    dim, h, Mgb = len(cells), 0.5, 0.4
+    mesh = CartesianMesh(cells, (0.0,) * dim, tuple(h * c for c in cells))
+    op = SinteringOperatorGeneric(mesh, G, FreeEnergyParams(), MobilityParams(Mgb=Mgb))
+    nn = [c + 1 for c in cells]
+    x = np.arange(nn[0])
+    u = np.zeros(nn[::-1] + [G + 2])
+    u[..., 0], u[..., 1], u[..., 2] = 1.0, h * x, 1.0
+    src = np.zeros_like(u)
+    src[..., 2], src[..., 3] = 1.0, 1e-5
+    want = np.ones(nn[::-1]) * np.where(x == 0, -1.0, np.where(x == cells[0], 1.0, 0.0))
+    for d in range(1, dim):
+        w = np.full(nn[d], h)
+        w[0] = w[-1] = h / 2
+        want *= w.reshape([-1 if a == dim - 1 - d else 1 for a in range(dim)])
+    want *= 2 * Mgb * 1e-5
+    op.fill_quadrature_point_values(dev(u.ravel()))
+    for dtype, eps in ((torch.float64, 2.0**-53), (torch.float32, 2.0**-24)):
+        dst = op.initialize_dof_vector(dtype)
+        op.vmult(dst, dev(src.ravel()).to(dtype))
+        got = host(dst).reshape(nn[::-1] + [G + 2])[..., 0]
+        rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+        assert rel <= 64 * eps, (dtype, rel)
