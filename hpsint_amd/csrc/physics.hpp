@@ -226,12 +226,15 @@ namespace hps
     T kj[3], kmu[3], keta[3], gsj[3];
   };
 
-  // scalar mobility (MobilityScalar::apply_M, S/mobility.h:441-472) from p = c
-  // (1 - c) and sum_{j < i} eta_i eta_j
+  // scalar mobility (MobilityScalar::apply_M, S/mobility.h:441-472) with
+  // pairs = sum_{j < i} eta_i eta_j.  (Two squares: the square of c (1 - c) would
+  // double that product's rounding.)
   template <typename T, typename PP>
-  __device__ __forceinline__ T scalar_mobility(const PP &pp, T c, T p, T pairs)
+  __device__ __forceinline__ T scalar_mobility(const PP &pp, T c, T pairs)
   {
-    return T(pp.Mvap) + pp_dM<T>(pp) * phi_clamped(c) + pp_Ms4<T>(pp) * (p * p) + pp_Mgb2<T>(pp) * pairs;
+    const T c1 = T(1.0) - c;
+    return T(pp.Mvap) + pp_dM<T>(pp) * phi_clamped(c) + pp_Ms4<T>(pp) * ((c * c) * (c1 * c1)) +
+           pp_Mgb2<T>(pp) * pairs;
   }
 
   // c-row coefficients of the scalar-mobility tangent
@@ -263,9 +266,118 @@ namespace hps
         sv += v[2 + i];
       }
     const T p    = c * (T(1.0) - c);
-    M            = scalar_mobility(pp, c, p, pairs);
+    M            = scalar_mobility(pp, c, pairs);
     const T dMdc = p * (pp_dM30<T>(pp) * p + pp_Ms8<T>(pp) * (T(1.0) - T(2.0) * c));
     s            = dMdc * v[0] + pp_Mgb2<T>(pp) * factor;
+  }
+
+  // The value rows term by term (S/operator_sintering_generic.h:104-190),
+  // with more operations than tangent_values_collected.  For the FP64 Q2 tile
+  // march, which waits for memory, not for the VALU: the collected form gained
+  // it nothing, and with its derived products in the argument block it took
+  // 3.58 instead of 3.42 ms (96^3, 10 order parameters, tensorial).
+  template <int G, typename T, typename PP>
+  __device__ __forceinline__ void tangent_values_by_term(const PP &pp, T c, const T *etas,
+                                                         const T *v, T *vr)
+  {
+    const T A = T(pp.A), B = T(pp.B), L = T(pp.L), w0 = T(pp.w0);
+    T       S2 = T(0.0);
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      S2 += etas[i] * etas[i];
+    vr[0] = v[0] * w0;
+    const T d2f_dc2 = T(2.0) * A * (c * c) + T(4.0) * A * c * (T(2.0) * c - T(2.0)) +
+                      T(2.0) * A * ((-c + T(1.0)) * (-c + T(1.0))) + T(2.0) * B;
+    T vmu = T(pp.w_alg) * v[1] - d2f_dc2 * v[0];
+    T d2f_dcdeta[G > 0 ? G : 1];
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      {
+        d2f_dcdeta[i] = (B * T(12.0)) * etas[i] * (etas[i] - T(1.0));
+        vmu -= d2f_dcdeta[i] * v[i + 2];
+      }
+    vr[1] = vmu;
+
+    // 3) eta rows
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      {
+        const T e        = etas[i];
+        const T d2f_de2  = B * (T(12.0) - T(12.0) * c + T(2.0) * e * (T(12.0) * c - T(24.0)) +
+                               T(24.0) * (e * e) + T(12.0) * S2);
+        vr[i + 2] = v[i + 2] * w0 + L * (d2f_dcdeta[i] * v[0] + d2f_de2 * v[i + 2]);
+      }
+    // apply_d2f_detaidetaj, S/free_energy.h:234-252
+    if constexpr (G > 1)
+      {
+        T temp = etas[0] * v[2];
+#pragma unroll
+        for (int i = 1; i < G; ++i)
+          temp += etas[i] * v[2 + i];
+        const T f = L * T(24.0) * B;
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+          vr[2 + i] += f * etas[i] * (temp - etas[i] * v[2 + i]);
+      }
+  }
+
+  // Value rows with the derivatives of the free energy
+  // (S/free_energy.h:37-176, 234-252) collected by powers of eta_i:
+  //   f_cc = 12 A c (c - 1) + 2 A + 2 B,  f_c,eta_i = 12 B eta_i (eta_i - 1),
+  //   f_eta_i,eta_i = 12 B (1 - c + S2) + 24 B (c - 2) eta_i + 24 B eta_i^2,
+  //   f_eta_i,eta_j = 24 B eta_i eta_j;
+  // the eta_i^2 part of the diagonal is the j = i term of
+  // 24 B eta_i sum_j eta_j deta_j.  The terms of a row that cancel in a grain
+  // (24 B (c - 2) eta_i deta_i and that sum) meet before anything is added to
+  // them, and w0 deta_i comes last: FP32 rms errors are 0.7-1.0 times those of the
+  // terms one by one in grains, at their boundaries and surfaces, for w0 from 0
+  // to 1000 (2 order parameters: up to 1.04 with w0 = 0).  With up to 5
+  // order parameters that takes a row of seven operations, in units of 12 B L;
+  // with more, five suffice.  (Four operations, with w0 in the factor of deta_i
+  // and the sum last, had 0.95-1.3 times the errors.)  Tangent with four / as
+  // here / seven for all, us: 128^3 FP64 with 4, 8: 317 / 322 / 322, 571 / 578 /
+  // 581; 160^3 FP64 with 12: 1618 / 1652 / 1664; 192^3 FP32 with 8: 1028 /
+  // 1050 / 1064.  (One order parameter: term by term.)
+  template <int G, typename T, typename PP>
+  __device__ __forceinline__ void tangent_values_collected(const PP &pp, T c, const T *etas,
+                                                           const T *v, T *vr)
+  {
+    const T w0 = T(pp.w0);
+    T       w = etas[0] * v[2], S2 = etas[0] * etas[0], ev = w, e2v = etas[0] * w;
+#pragma unroll
+    for (int i = 1; i < G; ++i)
+      {
+        S2 += etas[i] * etas[i];
+        w = etas[i] * v[2 + i];
+        ev += w;
+        e2v += etas[i] * w;
+      }
+    const T fcc = pp_A2B2<T>(pp) - pp_A12<T>(pp) * (c * (T(1.0) - c));
+    vr[0]       = v[0] * w0;
+    vr[1]       = (T(pp.w_alg) * v[1] - pp_B12<T>(pp) * (e2v - ev)) - fcc * v[0];
+    const T s   = (T(1.0) - c) + S2;
+    if constexpr (G <= 5)
+      {
+        const T b = T(2.0) * c - T(4.0), ev2 = T(2.0) * ev;
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+          {
+            const T e = etas[i], x = v[2 + i];
+            const T t = s * x + e * ((b * x + ev2) + v[0] * (e - T(1.0)));
+            vr[2 + i] = w0 * x + pp_BL12<T>(pp) * t;
+          }
+      }
+    else
+      {
+        const T a = pp_BL12<T>(pp) * s, b = pp_BL24<T>(pp) * (c - T(2.0));
+        const T c0 = pp_BL12<T>(pp) * v[0], f0 = pp_BL24<T>(pp) * ev - c0;
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+          {
+            const T e = etas[i], x = v[2 + i];
+            vr[2 + i] = w0 * x + (a * x + e * (b * x + (c0 * e + f0)));
+          }
+      }
   }
 
   // qsum (optional, tensorial only): sum_i deta_i Q_i formed by the caller,
@@ -402,32 +514,11 @@ namespace hps
         gr[i + 2][d] = Lkp * g[i + 2][d];
     if constexpr (!VALS)
       return;
-    // Value rows with the derivatives of the free energy
-    // (S/free_energy.h:37-176, 234-252) collected by powers of eta_i:
-    //   f_cc = 12 A c (c - 1) + 2 A + 2 B,  f_c,eta_i = 12 B eta_i (eta_i - 1),
-    //   f_eta_i,eta_i = 12 B (1 - c + S2) + 24 B (c - 2) eta_i + 24 B eta_i^2,
-    //   f_eta_i,eta_j = 24 B eta_i eta_j;
-    // the eta_i^2 part of the diagonal is the j = i term of
-    // 24 B eta_i sum_j eta_j deta_j, so a row costs four operations:
-    //   (b eta_i + a) deta_i + eta_i (c0 eta_i + 24 B L sum_j eta_j deta_j - c0),
-    //   a = w0 + 12 B L (1 - c + S2), b = 24 B L (c - 2), c0 = 12 B L dc
-    const T e0 = G > 0 ? etas[0] : T(0.0);
-    T       w = G > 0 ? e0 * v[2] : T(0.0), S2 = e0 * e0, ev = w, e2v = e0 * w;
-#pragma unroll
-    for (int i = 1; i < G; ++i)
-      {
-        S2 += etas[i] * etas[i];
-        w = etas[i] * v[2 + i];
-        ev += w;
-        e2v += etas[i] * w;
-      }
-    const T fcc = pp_A12<T>(pp) * (c * (c - T(1.0))) + pp_A2B2<T>(pp);
-    vr[1]       = T(pp.w_alg) * v[1] - fcc * v[0] - pp_B12<T>(pp) * (e2v - ev);
-    const T a = w0 + pp_BL12<T>(pp) * ((T(1.0) - c) + S2), b = pp_BL24<T>(pp) * (c - T(2.0));
-    const T c0 = pp_BL12<T>(pp) * v[0], f0 = pp_BL24<T>(pp) * ev - c0;
-#pragma unroll
-    for (int i = 0; i < G; ++i)
-      vr[i + 2] = (b * etas[i] + a) * v[i + 2] + etas[i] * (c0 * etas[i] + f0);
+    // value rows
+    if constexpr (G <= 1)
+      tangent_values_by_term<G>(pp, c, etas, v, vr);
+    else
+      tangent_values_collected<G>(pp, c, etas, v, vr);
   }
 
   template <int DIM, int G, bool TENS, typename T, typename PP>
@@ -444,56 +535,6 @@ namespace hps
   // stream one component at a time use these pieces; tangent_qp above is
   // their composition.
   // ------------------------------------------------------------------
-  // The value rows term by term (S/operator_sintering_generic.h:104-190),
-  // with more operations than the collected form of tangent_qp_rows: the FP64
-  // Q2 tile march waits for memory, not for the VALU.  The collected form gained
-  // it nothing, and with its derived products in the argument block it took
-  // 3.58 instead of 3.42 ms (96^3, 10 order parameters, tensorial).
-  template <int G, typename T, typename PP>
-  __device__ __forceinline__ void tangent_values_by_term(const PP &pp, T c, const T *etas,
-                                                         const T *v, T *vr)
-  {
-    const T A = T(pp.A), B = T(pp.B), L = T(pp.L), w0 = T(pp.w0);
-    T       S2 = T(0.0);
-#pragma unroll
-    for (int i = 0; i < G; ++i)
-      S2 += etas[i] * etas[i];
-    vr[0] = v[0] * w0;
-    const T d2f_dc2 = T(2.0) * A * (c * c) + T(4.0) * A * c * (T(2.0) * c - T(2.0)) +
-                      T(2.0) * A * ((-c + T(1.0)) * (-c + T(1.0))) + T(2.0) * B;
-    T vmu = T(pp.w_alg) * v[1] - d2f_dc2 * v[0];
-    T d2f_dcdeta[G > 0 ? G : 1];
-#pragma unroll
-    for (int i = 0; i < G; ++i)
-      {
-        d2f_dcdeta[i] = (B * T(12.0)) * etas[i] * (etas[i] - T(1.0));
-        vmu -= d2f_dcdeta[i] * v[i + 2];
-      }
-    vr[1] = vmu;
-
-    // 3) eta rows
-#pragma unroll
-    for (int i = 0; i < G; ++i)
-      {
-        const T e        = etas[i];
-        const T d2f_de2  = B * (T(12.0) - T(12.0) * c + T(2.0) * e * (T(12.0) * c - T(24.0)) +
-                               T(24.0) * (e * e) + T(12.0) * S2);
-        vr[i + 2] = v[i + 2] * w0 + L * (d2f_dcdeta[i] * v[0] + d2f_de2 * v[i + 2]);
-      }
-    // apply_d2f_detaidetaj, S/free_energy.h:234-252
-    if constexpr (G > 1)
-      {
-        T temp = etas[0] * v[2];
-#pragma unroll
-        for (int i = 1; i < G; ++i)
-          temp += etas[i] * v[2 + i];
-        const T f = L * T(24.0) * B;
-#pragma unroll
-        for (int i = 0; i < G; ++i)
-          vr[2 + i] += f * etas[i] * (temp - etas[i] * v[2 + i]);
-      }
-  }
-
   // BY_TERM: tangent_values_by_term
   template <int DIM, int G, bool TENS, bool BY_TERM = false, typename T, typename PP>
   __device__ __forceinline__ void tangent_values(const PP &pp, const T *lin,
@@ -582,7 +623,7 @@ namespace hps
             pairs += etas[i] * sum;
             sum += etas[i];
           }
-        const T M = scalar_mobility(pp, c, c * (T(1.0) - c), pairs);
+        const T M = scalar_mobility(pp, c, pairs);
 #pragma unroll
         for (int d = 0; d < DIM; ++d)
           gr[0][d] = M * g[1][d];
@@ -749,7 +790,7 @@ namespace hps
         pairs += etas[i] * sum;
         sum += etas[i];
       }
-    const T M = scalar_mobility(pp, c, c * (T(1.0) - c), pairs);
+    const T M = scalar_mobility(pp, c, pairs);
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
       out[d] = M * g1[d];
