@@ -83,38 +83,31 @@ namespace hps
   } // namespace
 
   // ---------------------------------------------------------------- assembly
-  // one thread per cell of parity colour `par`; the cell's 2^DIM x 2^DIM
-  // element matrix (2x2 per node pair) is added to the rows of its nodes
-  template <int DIM>
+  // 2D: one thread per cell of parity colour `par`; the cell's 4 x 4 element
+  // matrix (2x2 per node pair) is added to the rows of its nodes
   __global__ void __launch_bounds__(256)
-    k_ch_assemble(const ChParams cp, int par, const double *__restrict__ cache,
-                  double *__restrict__ A)
+    k_ch_assemble_2d(const ChParams cp, int par, const double *__restrict__ cache,
+                     double *__restrict__ A)
   {
-    constexpr int NV = 1 << DIM;
-    constexpr int S  = Sten<DIM>::S;
-    const int     px = par & 1, py = (par >> 1) & 1, pz = (par >> 2) & 1;
+    constexpr int NV = 4;
+    const int     px = par & 1, py = par >> 1;
     const int     mx = (cp.nc[0] - px + 1) / 2, my = (cp.nc[1] - py + 1) / 2;
-    const int     mz = DIM == 3 ? (cp.nc[2] - pz + 1) / 2 : 1;
     const int64_t i  = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (int64_t)mx * my * mz)
+    if (i >= (int64_t)mx * my)
       return;
     const int cx = px + 2 * (int)(i % mx);
-    const int cy = py + 2 * (int)((i / mx) % my);
-    const int cz = DIM == 3 ? pz + 2 * (int)(i / ((int64_t)mx * my)) : 0;
+    const int cy = py + 2 * (int)(i / mx);
 
     // the cell's place in the cache (lane order of the Q1 kernels: tiles of
-    // tx x ty cells, tz layers along the last direction)
-    const int cm   = DIM == 3 ? cz : cy;  // march direction
-    const int cyy  = DIM == 3 ? cy : 0;
-    const int64_t tile =
-      (int64_t)(cx / cp.tx) + (int64_t)cp.nt[0] * ((cyy / cp.ty) + (int64_t)cp.nt[1] * (cm / cp.tz));
-    const int     layer = cm % cp.tz;
-    const int     lane0 = (((cyy % cp.ty) * cp.tx) + (cx % cp.tx)) << DIM;
+    // tx cells, tz rows along y)
+    const int64_t tile  = (cx / cp.tx) + (int64_t)cp.nt[0] * cp.nt[1] * (cy / cp.tz);
+    const int     layer = cy % cp.tz;
+    const int     lane0 = (cx % cp.tx) << 2;
     const double *cl    = cache + ((tile * cp.tz + layer) * cp.nf) * (int64_t)cp.nt_lanes;
 
     const double A_ = cp.pp.A, B_ = cp.pp.B;
     // quadrature-point coefficients of the Cahn-Hilliard block
-    double Mq[NV], dMq[NV], d2q[NV], lmu[NV][3];
+    double Mq[NV], dMq[NV], d2q[NV], lmu[NV][2];
 #pragma unroll
     for (int q = 0; q < NV; ++q)
       {
@@ -127,8 +120,8 @@ namespace hps
             eta_sum += e;
           }
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-          lmu[q][d] = d < DIM ? cl[(1 + cp.G + d) * (int64_t)cp.nt_lanes + lane0 + q] : 0.0;
+        for (int d = 0; d < 2; ++d)
+          lmu[q][d] = cl[(1 + cp.G + d) * (int64_t)cp.nt_lanes + lane0 + q];
         const double phi    = dmin(1.0, dmax(0.0, c * c * c * (10.0 - 15.0 * c + 6.0 * c * c)));
         Mq[q]               = cp.pp.Mvol * phi + cp.pp.Mvap * (1.0 - phi) +
                 cp.pp.Msurf * 4.0 * c * c * (1.0 - c) * (1.0 - c) + (2.0 * cp.pp.Mgb) * eta_ij;
@@ -146,11 +139,9 @@ namespace hps
 #pragma unroll 1
     for (int k = 0; k < NV; ++k)
       {
-        const int     kx = cx + (k & 1), ky = cy + ((k >> 1) & 1);
-        const int     kz = DIM == 3 ? cz + ((k >> 2) & 1) : 0;
         // the colour of corner k: the cell parity flipped by the corner's
         // bits (uniform)
-        const RowRef<double> ra = row_of(cp, A, par ^ k, kx, ky, kz);
+        const RowRef<double> ra = row_of(cp, A, par ^ k, cx + (k & 1), cy + (k >> 1), 0);
 #pragma unroll
         for (int m = 0; m < NV; ++m)
           {
@@ -158,19 +149,19 @@ namespace hps
 #pragma unroll
             for (int q = 0; q < NV; ++q)
               {
-                double vk = 1.0, vm = 1.0, gk[3], gm[3];
+                double vk = 1.0, vm = 1.0, gk[2], gm[2];
 #pragma unroll
-                for (int d = 0; d < DIM; ++d)
+                for (int d = 0; d < 2; ++d)
                   {
                     vk *= (((k >> d) & 1) == ((q >> d) & 1)) ? sa : sb;
                     vm *= (((m >> d) & 1) == ((q >> d) & 1)) ? sa : sb;
                   }
 #pragma unroll
-                for (int d = 0; d < DIM; ++d)
+                for (int d = 0; d < 2; ++d)
                   {
                     double fk = ((k >> d) & 1) ? 1.0 : -1.0, fm = ((m >> d) & 1) ? 1.0 : -1.0;
 #pragma unroll
-                    for (int e = 0; e < DIM; ++e)
+                    for (int e = 0; e < 2; ++e)
                       if (e != d)
                         {
                           fk *= (((k >> e) & 1) == ((q >> e) & 1)) ? sa : sb;
@@ -181,7 +172,7 @@ namespace hps
                   }
                 double gg = 0.0, mug = 0.0;
 #pragma unroll
-                for (int d = 0; d < DIM; ++d)
+                for (int d = 0; d < 2; ++d)
                   {
                     gg += gm[d] * gk[d];
                     mug += lmu[q][d] * gk[d];
@@ -192,9 +183,8 @@ namespace hps
                 a2 += -d2q[q] * vv - cp.pp.kappa_c * gg;
                 a3 += cp.pp.w_alg * vv;
               }
-            const int dx = (m & 1) - (k & 1), dy = ((m >> 1) & 1) - ((k >> 1) & 1);
-            const int dz = DIM == 3 ? ((m >> 2) & 1) - ((k >> 2) & 1) : 0;
-            const int s4 = 4 * Sten<DIM>::index(dx, dy, dz);
+            const int dx = (m & 1) - (k & 1), dy = (m >> 1) - (k >> 1);
+            const int s4 = 4 * Sten<2>::index(dx, dy, 0);
             ra[s4 + 0] += jxw * a0;
             ra[s4 + 1] += jxw * a1;
             ra[s4 + 2] += jxw * a2;
@@ -293,7 +283,8 @@ namespace hps
     const int z0 = (b / (nwx * nwy)) * zn, z1 = min(z0 + zn, cp.nn[2]);
     const bool in_cell = gx >= 0 && gx < cp.nc[0] && gy >= 0 && gy < cp.nc[1];
     const bool own     = ci > 0 && cj > 0 && gx < cp.nn[0] && gy < cp.nn[1];
-    // the cell's place in the cache (as k_ch_assemble)
+    // the cell's place in the cache (lane order of the Q1 kernels: tiles of
+    // tx x ty cells, tz layers along z)
     const int64_t ntl   = cp.nt_lanes;
     const int64_t tile0 = in_cell ? (gx / cp.tx) + (int64_t)cp.nt[0] * (gy / cp.ty) : 0;
     const int     lane0 = in_cell ? ((gy % cp.ty) * cp.tx + gx % cp.tx) << 3 : 0;
@@ -534,7 +525,7 @@ namespace hps
     const int     cz = DIM == 3 ? pz + 2 * (int)(i / ((int64_t)mx * my)) : 0;
     if (valid)
       {
-        // the cell's place in the cache (as k_ch_assemble)
+        // the cell's place in the cache (as k_ch_assemble_2d)
         const int     cm    = DIM == 3 ? cz : cy;
         const int     cyy   = DIM == 3 ? cy : 0;
         const int64_t tile  = (int64_t)(cx / cp.tx) +
@@ -1163,7 +1154,7 @@ namespace hps
         if (cp.tens)
           ch_assemble_tens(cp, par, n, cache, A, s);
         else
-          k_ch_assemble<2><<<blocks_for(n), 256, 0, s>>>(cp, par, cache, A);
+          k_ch_assemble_2d<<<blocks_for(n), 256, 0, s>>>(cp, par, cache, A);
       }
   }
 
