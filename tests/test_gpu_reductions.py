@@ -161,17 +161,23 @@ def test_orthogonalise_zero():
         call_orthogonalise(op, np.zeros((33, 8)), np.zeros(8), torch.float64)
 
 
-@pytest.mark.parametrize("cells,G,tens", [
-    ((24, 24, 24), 4, False),   # fewest layers per tile
-    ((24, 24, 24), 5, False),   # fewest of five and more order parameters
-    ((64, 40, 33), 3, False),   # between
-    ((96, 96, 70), 2, False),   # unchanged
-    ((160, 81), 2, False), ((33, 500), 3, True), ((17, 9, 30), 3, True)])
-def test_tile_depth_of_small_meshes(monkeypatch, cells, G, tens):
-    """tangent, residual and diagonal with the depth chosen for the mesh against
-    16 layers.  Only the order in which the cells of a node are added differs:
-    8 (2D 4) cell sums, 8 roundings of half an ulp of values that may cancel to
-    about a tenth: 1e-14 in the norm"""
+# layers: the deepest of 16, 8, 4 and (up to 4 order parameters) 2 that gives 768
+# tiles of 8 x 4 cells (2D: 64) and that many layers, or the shallowest
+@pytest.mark.parametrize("cells,G,tens,layers", [
+    ((24, 24, 24), 4, False, 2),    # fewest layers per tile
+    ((24, 24, 24), 5, False, 4),    # fewest of five and more order parameters
+    ((64, 40, 45), 3, False, 4),    # 960 tiles; 480 with 8 layers
+    ((64, 64, 64), 4, False, 8),    # 1024; 512 with 16
+    ((64, 64, 64), 7, False, 8),
+    ((96, 96, 48), 2, False, 16),   # 864: unchanged
+    ((160, 81), 2, False, 2), ((33, 500), 3, True, 2), ((17, 9, 30), 3, True, 2),
+    ((2000, 368), 2, False, 8)])    # 32 columns, 46 rows of tiles; 23 with 16 layers
+def test_tile_depth_of_small_meshes(monkeypatch, cells, G, tens, layers):
+    """tangent, residual and diagonal with the depth chosen for the mesh: bit for
+    bit those of the expected depth, and against 16 layers.  Only the order in
+    which the cells of a node are added differs there: 8 (2D 4) cell sums, 8
+    roundings of half an ulp of values that may cancel to about a tenth: 1e-14 in
+    the norm"""
     dim = len(cells)
     mesh = CartesianMesh(cells, (0.0,) * dim, tuple(0.5 * c for c in cells))
     nn = int(np.prod([c + 1 for c in cells]))
@@ -197,7 +203,11 @@ def test_tile_depth_of_small_meshes(monkeypatch, cells, G, tens):
         return out
 
     got = results()
+    monkeypatch.setenv("HPSINT_AMD_TILE_M", str(layers))
+    for g, r in zip(got, results()):
+        assert np.array_equal(g, r)
     monkeypatch.setenv("HPSINT_AMD_TILE_M", "16")
     ref = results()
+    assert layers == 16 or not np.array_equal(got[0], ref[0])
     for g, r, tol in zip(got, ref, (1e-14, 1e-14 * 2.0**29, 1e-14, 1e-14)):
         assert np.linalg.norm(g - r) <= tol * np.linalg.norm(r)
