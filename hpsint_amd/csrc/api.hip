@@ -375,14 +375,16 @@ extern "C" int hps_create(const hps_params *prm, hps_operator *out)
             op->zcol_mz = m * TZ;
             break;
           }
-      // FP64 tangent with 6 or 7 order parameters: only with two rounds of the
-      // marches that run at once; below that the emptier last round costs what
-      // the lanes save.  Corner lanes / z-column lanes, us, with 5, 6, 7 order
-      // parameters: 128^3 417 / 375, 456 / 422, 523 / 470; 160 x 150 x 170
-      // 808 / 737, 892 / 821, 1013 / 926; 90^3 (864 marches) 171 / 164,
-      // 184 / 187, 209 / 208; 61 x 75 x 67 (400) 71.9 / 71.7, 80 / 84,
-      // 95 / 95; 8 at 128^3 568 / 562 (spills), smaller meshes up to 18 %
-      // slower.
+      // FP64 tangent: always with up to 5 order parameters, with 6 or 7 only on
+      // meshes of two rounds of the marches that run at once.  Corner lanes /
+      // z-column lanes, us, at the tile depth that the mesh gets: with 5 8^3
+      // 18.4 / 18.9, 24^3 21.8 / 22.7, 40^3 26.7 / 24.5, 64^3 56 / 50, 61 x 75
+      // x 67 (8 layers per tile, 720 marches) 73 / 71, 90^3 (864) 173 / 164,
+      // 128^3 424 / 379; with 6, 7 24^3 22.9 / 24.2, 25.8 / 26.1, 61 x 75 x 67
+      // 84 / 85, 103 / 101, 72^3 (405) 104 / 105, 117 / 116, 90^3 192 / 189,
+      // 216 / 212, 128^3 476 / 436, 540 / 486 (64^3, 1024 tiles of 8 layers in
+      // 512 marches, would gain: 62 / 56, 73 / 65); 8 at 128^3 568 / 562
+      // (spills), smaller meshes up to 18 % slower.
       const int64_t marches = (int64_t)kp.nt[0] * op->ntz1 *
                               ((ncm + op->zcol_mz - 1) / op->zcol_mz);
       op->zcol = zc && (G <= 5 || (G <= hps::ZCOL_MAX_G && marches >= 4 * (int64_t)cus));
@@ -674,9 +676,10 @@ extern "C" int hps_residual(hps_operator op, int wtd, double *dst, const double 
   const int w = (wtd == 2 && op->kp.order == 0) ? 1 : wtd;
   // z-column lanes: with 5 and 6 order parameters the second history vector
   // costs them more than the corner lanes.  Corner / z-column lanes, us, one
-  // history vector: 128^3 409 / 365 and 493 / 412, 90^3 159 / 149 and 194 /
-  // 172, 61 x 75 x 67 78.8 / 78.7 and 93 / 89 (7: 103 / 110); two: 128^3 448 /
-  // 455 and 532 / 500, 61 x 75 x 67 84 / 94 and 99 / 105.
+  // history vector: 8^3 20.0 / 19.9 and 22.2 / 21.6, 40^3 29 / 25 and 32 / 28,
+  // 61 x 75 x 67 79 / 78 and 93 / 88, 90^3 160 / 148 and 195 / 170, 128^3 418 /
+  // 364 and 498 / 410 (7, 61 x 75 x 67: 103 / 110); two: 128^3 448 / 455 and
+  // 532 / 500, 61 x 75 x 67 84 / 94 and 99 / 105 (there with 16 layers per tile).
   const bool zres = op->zcol_residual && !op->cut_active &&
                     (op->n_grains <= 4 || w < 2 || op->kp.order < 2);
   if (op->q2)

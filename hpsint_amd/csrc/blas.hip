@@ -3,8 +3,9 @@
 // DynamicBlockVector operations (I/lac/dynamic_block_vector.h:346-537) on
 // the component-interleaved storage, the inverse-diagonal and inverse
 // node-block applies (I/lac/preconditioners.h:160-318) and the layout
-// conversions (I/numerics/vector_tools.h:40-100).  Reductions use a fixed
-// grid and a fixed second-pass order, so results do not depend on timing.
+// conversions (I/numerics/vector_tools.h:40-100).  A reduction's grid is a
+// function of the length alone (red_blocks) and its second pass has a fixed
+// order, so results do not depend on timing.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

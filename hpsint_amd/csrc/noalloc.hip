@@ -66,8 +66,9 @@ extern "C" int hps_multi_dot_noalloc(void *stream, int64_t n, int k, const doubl
   double *ptr = nullptr;
   if (int r = scratch_of_current_device(&ptr))
     return r;
-  // the partial rows are written in full by every call (each reduction
-  // block stores its k sums, empty blocks store zeros): nothing to clear
+  // every call writes the first red_blocks(n) partial rows in full and its
+  // second pass reads no others (rows beyond them keep an earlier call's sums):
+  // nothing to clear
   hps::blas_multi_dot(static_cast<hipStream_t>(stream), n, k, V, w, ptr, h);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess)
