@@ -220,8 +220,9 @@ namespace hps
   // sum-factorised butterflies for every k but for the gradients' signs.
   // (Adding each cell's element matrix to its rows, in 8 cell-parity passes,
   // read and wrote a row 8 times.)
-  // Bound: FP64 VALU issue and the 864 bytes written per node; 129^3 nodes, 4
-  // order parameters: 1.06 ms (4.6 with the passes; the bytes take 0.6).
+  // Bound: latency at 2 waves per SIMD (VALU slots 26 % busy) over the 864 bytes
+  // written per node and the cache; 129^3 nodes, 4 order parameters: 1.06 ms (4.6
+  // with the passes; the bytes take 0.6 at the copy rate).
   namespace cha
   {
     constexpr int WX = 16, WY = 8, OX = WX - 1, OY = WY - 1, NT = WX * WY;

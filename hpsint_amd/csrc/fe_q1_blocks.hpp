@@ -84,7 +84,8 @@ namespace hps
   // in registers, x and y by DPP butterflies, the four cells around a node
   // through LDS.  Sweep [F0, F1) forms those fields and writes the entries
   // made of them.
-  // Bound: VALU issue at 2 waves/SIMD; 1.88 M nodes, 8 order parameters, FP32:
+  // Bound: VALU issue (slots 71 % busy) and HBM (3.7 of a copy's 4.8 TB/s) at 2
+  // waves/SIMD; 1.88 M nodes, 8 order parameters, FP32:
   // 0.78 ms where ten q1_probe launches, their fix-ups and the conversion to
   // FP64 took 4.1 ms (the 1.5 GB written take 0.31 ms at the copy rate).
   template <int G, typename T, int F0, int F1>

@@ -49,9 +49,10 @@ namespace hps
   // direction; the results of a lane's node stay in registers until its block
   // is written.  The flux and stiffness sums come first, while the cache
   // fields are held; the mass sums need c and eta_i only.
-  // Bound: VALU issue at 2 waves/SIMD (7 k of 10 k instructions per cell
-  // pair); 40 x 45 x 37 cells, 10 order parameters, FP64 tensorial: 1.6 ms, of
-  // which the 3.5 GB of the colour passes take 0.73 ms at the copy rate (3.7 ms
+  // Bound: latency at 2 waves/SIMD, of the LDS passes (1000 LDS of 8 k
+  // instructions per wave; VALU slots 21 % busy) and of the blocks that the colour
+  // passes read back; 40 x 45 x 37 cells, 10 order parameters, FP64 tensorial:
+  // 1.6 ms, 4.6 GB moved (0.96 ms at the copy rate; one write is 0.64 GB) (3.7 ms
   // with one column at a time; 1.95 ms with every lane storing its own block,
   // 16 bytes per line).
   template <int DIM, int G, bool TENS, typename T>

@@ -13,7 +13,8 @@
 //
 // Measured at 161^3 nodes, 12 order parameters, with the increment norm: 1.97
 // ms (k_fields 0.32, at 4.9 TB/s; k_infer 1.45, 0.88 of it VALU issue, most
-// of that the 384 tanh per node; its MFMA 0.24).  Feature, layer and
+// of that the 384 tanh per node; its MFMA 0.24; the rest is waiting for the
+// gathers at 2 waves/SIMD).  Feature, layer and
 // correction kernels one after the other, with a row of 272 features per node
 // in memory, took 13.4 ms; one kernel whose waves shared a tile's features
 // and activations through LDS 3.1 ms (15 barriers per tile, 2 waves/SIMD).
