@@ -222,7 +222,8 @@ int hps_multi_axpy_norm(hps_operator op, int64_t n, int k, const double *V,
 /* w made orthogonal to the k (1..32) vectors of V (orthonormal, back to back)
  * by classical Gram-Schmidt and normalised: on return the old w is sum_j h[j]
  * V_j + norm w, |w| = 1 (w = 0 if norm is 0).  A second pass runs when the first
- * leaves less than half of w's norm. */
+ * leaves less than half of w's norm.  h and norm are returned; w is ready in the
+ * stream's order. */
 int hps_orthogonalise(hps_operator op, int64_t n, int k, const double *V, double *w, double *h,
                       double *norm);
 /* y += sum_{j<k} a[j] V_j (the GMRES solution update x += V y; a on the
